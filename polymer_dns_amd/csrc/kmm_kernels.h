@@ -282,15 +282,18 @@ hipError_t launch_audit_residual(const float* pred, const float* ref, size_t n, 
 // learned closure (kmm_mlp.hip)
 int mlp_param_count();
 int mlp_wb_count();
-int mlp_fb_blocks(int n);
+// floats of training workspace for n samples (inputs, deltas, gradient and loss partials)
+size_t mlp_train_ws(int n);
 hipError_t launch_mlp_infer(int n, const float* X, float* Y, const void* wb, const float* par, const float* norm,
                             int act, hipStream_t s);
 hipError_t launch_mlp_pack(const float* par, void* wb, hipStream_t s);
-// mode bit 0: bf16 rounding as in inference; bit 1: GELU (else ReLU)
+// loss and gradient; mode bit 0: bf16 rounding as in inference; bits 1-2: activation
 hipError_t launch_mlp_grad(int n, const float* X, const float* T, const float* par, const float* norm, int mode,
-                           float* gpart, float* lpart, float* g, float* loss, hipStream_t s);
-hipError_t launch_mlp_adam(float* par, float* m, float* v, const float* g, float lr, int t, void* wb,
-                           hipStream_t s);
+                           float* ws, float* g, float* loss, hipStream_t s);
+// the same followed by Adam step t on par and the refresh of the bf16 copy wb
+hipError_t launch_mlp_train_step(int n, const float* X, const float* T, float* par, const float* norm, int mode,
+                                 float* ws, float* g, float* loss, float* m, float* v, float lr, int t, void* wb,
+                                 hipStream_t s);
 hipError_t launch_gradv(int ny, int P, int nz, double alpha, double beta, double dyde, const double2* u,
                         const double2* v, const double2* w, double2* const* out, hipStream_t s);
 // swirl strength of n velocity-gradient tensors; g[k*n + j] = component k

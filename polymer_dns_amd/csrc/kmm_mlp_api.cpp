@@ -25,8 +25,8 @@ struct kmm_mlp {
   int adam_t = 0;
   int act = 0;                      // hidden-layer activation: 0 ReLU, 1 GELU, 2 GELU (polynomial sigmoid)
   // scratch (grown on demand)
-  float *X = nullptr, *T = nullptr, *Y = nullptr, *gpart = nullptr, *lpart = nullptr, *loss = nullptr;
-  size_t capX = 0, capT = 0, capY = 0, capG = 0;
+  float *X = nullptr, *T = nullptr, *Y = nullptr, *ws = nullptr, *loss = nullptr;
+  size_t capX = 0, capT = 0, capY = 0, capW = 0;
 };
 
 static int mfail(int code, const std::string& msg) {
@@ -92,7 +92,7 @@ extern "C" int kmm_mlp_destroy(kmm_mlp* n) {
   if (!n) return KMM_OK;
   hipSetDevice(n->device);
   if (n->stream) hipStreamSynchronize(n->stream);
-  for (float* p : {n->par, n->m, n->v, n->g, n->norm, n->X, n->T, n->Y, n->gpart, n->lpart, n->loss})
+  for (float* p : {n->par, n->m, n->v, n->g, n->norm, n->X, n->T, n->Y, n->ws, n->loss})
     if (p) hipFree(p);
   if (n->wb) hipFree(n->wb);
   if (n->stream) hipStreamDestroy(n->stream);
@@ -158,17 +158,14 @@ extern "C" int kmm_mlp_grad(kmm_mlp* n, int npts, const float* X, const float* T
                             float* loss) {
   if (!n || npts <= 0 || !X || !T || !grad || !loss || (mode != 0 && mode != 1)) return mfail(KMM_E_ARG, "bad argument");
   MHIP(hipSetDevice(n->device));
-  const int nb = kmm::mlp_fb_blocks(npts);
   int r;
   if ((r = grow(&n->X, &n->capX, (size_t)npts * 22)) || (r = grow(&n->T, &n->capT, (size_t)npts * 6)) ||
-      (r = grow(&n->gpart, &n->capG, (size_t)nb * n->np)))
+      (r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(npts))))
     return r;
-  if (n->lpart) hipFree(n->lpart);
-  MHIP(hipMalloc((void**)&n->lpart, (size_t)nb * sizeof(float)));
   MHIP(hipMemcpyAsync(n->X, X, (size_t)npts * 22 * sizeof(float), hipMemcpyHostToDevice, n->stream));
   MHIP(hipMemcpyAsync(n->T, T, (size_t)npts * 6 * sizeof(float), hipMemcpyHostToDevice, n->stream));
-  MHIP(kmm::launch_mlp_grad(npts, n->X, n->T, n->par, n->norm, mode | (n->act << 1), n->gpart, n->lpart, n->g,
-                            n->loss, n->stream));
+  MHIP(kmm::launch_mlp_grad(npts, n->X, n->T, n->par, n->norm, mode | (n->act << 1), n->ws, n->g, n->loss,
+                            n->stream));
   MHIP(hipMemcpyAsync(grad, n->g, (size_t)n->np * sizeof(float), hipMemcpyDeviceToHost, n->stream));
   MHIP(hipMemcpyAsync(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
   MHIP(hipStreamSynchronize(n->stream));
@@ -188,13 +185,10 @@ extern "C" int kmm_mlp_train(kmm_mlp* n, int npts, const float* X, const float* 
   std::iota(perm.begin(), perm.end(), 0);
   std::mt19937_64 rng(seed);
   std::vector<float> bx((size_t)batch * 22), bt((size_t)batch * 6);
-  const int nb = kmm::mlp_fb_blocks(batch);
   int r;
   if ((r = grow(&n->X, &n->capX, (size_t)batch * 22)) || (r = grow(&n->T, &n->capT, (size_t)batch * 6)) ||
-      (r = grow(&n->gpart, &n->capG, (size_t)nb * n->np)))
+      (r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(batch))))
     return r;
-  if (n->lpart) hipFree(n->lpart);
-  MHIP(hipMalloc((void**)&n->lpart, (size_t)nb * sizeof(float)));
   int pos = npts;
   for (int s = 0; s < steps; ++s) {
     if (pos + batch > npts) {
@@ -209,9 +203,8 @@ extern "C" int kmm_mlp_train(kmm_mlp* n, int npts, const float* X, const float* 
     pos += batch;
     MHIP(hipMemcpyAsync(n->X, bx.data(), bx.size() * sizeof(float), hipMemcpyHostToDevice, n->stream));
     MHIP(hipMemcpyAsync(n->T, bt.data(), bt.size() * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    MHIP(kmm::launch_mlp_grad(batch, n->X, n->T, n->par, n->norm, 1 | (n->act << 1), n->gpart, n->lpart, n->g,
-                              n->loss, n->stream));
-    MHIP(kmm::launch_mlp_adam(n->par, n->m, n->v, n->g, lr, ++n->adam_t, n->wb, n->stream));
+    MHIP(kmm::launch_mlp_train_step(batch, n->X, n->T, n->par, n->norm, 1 | (n->act << 1), n->ws, n->g, n->loss, n->m,
+                                    n->v, lr, ++n->adam_t, n->wb, n->stream));
     if (losses) MHIP(hipMemcpyAsync(losses + s, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
     // the host buffers are reused by the next batch
     MHIP(hipStreamSynchronize(n->stream));
@@ -228,18 +221,13 @@ int kmm_mlp_train_device(kmm_mlp* n, int npts, const float* dX, const float* dT,
                          hipStream_t s) {
   if (!n || npts <= 0 || !dX || !dT || steps <= 0 || batch <= 0 || batch > npts || !(lr > 0.0f))
     return mfail(KMM_E_ARG, "bad argument");
-  const int nb = kmm::mlp_fb_blocks(batch);
   int r;
-  if ((r = grow(&n->gpart, &n->capG, (size_t)nb * n->np))) return r;
-  if (n->lpart) hipFree(n->lpart);
-  MHIP(hipMalloc((void**)&n->lpart, (size_t)nb * sizeof(float)));
+  if ((r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(batch)))) return r;
   const int nblocks = npts / batch;
   for (int k = 0; k < steps; ++k) {
     const size_t off = (size_t)(k % nblocks) * batch;
-    MHIP(kmm::launch_mlp_grad(batch, dX + off * 22, dT + off * 6, n->par, n->norm, 1 | (n->act << 1), n->gpart,
-                              n->lpart, n->g,
-                              n->loss, s));
-    MHIP(kmm::launch_mlp_adam(n->par, n->m, n->v, n->g, lr, ++n->adam_t, n->wb, s));
+    MHIP(kmm::launch_mlp_train_step(batch, dX + off * 22, dT + off * 6, n->par, n->norm, 1 | (n->act << 1), n->ws, n->g,
+                                    n->loss, n->m, n->v, lr, ++n->adam_t, n->wb, s));
   }
   return KMM_OK;
 }

@@ -122,3 +122,35 @@ def test_gelu_gradients_and_inference_match_oracle(kind):
     finally:
         M.ACT = "relu"
     net.close()
+
+
+# samples per block 16, four blocks in flight and 4096 samples per chunk of
+# the weight gradient: one sample, both sides of a block, of four blocks and
+# of a chunk, and two chunks
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 1025, 4096, 4097, 5000])
+def test_gradient_at_block_and_chunk_edges(n):
+    """Loss and FP32 gradient vs the oracle's FP64 ones.  Every value is a sum
+    of FP32 products over at most 128 inputs per layer and the n samples:
+    with rounding errors adding up like a random walk through five layers
+    forward and back, sqrt(10 * 128) * 2^-24 = 2e-6 of the gradient's norm;
+    the bound leaves a factor of five."""
+    net, nm = setup_net(seed=21)
+    net.set_activation("gelu_poly")
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 22)).astype(np.float32)
+    T = rng.standard_normal((n, 6)).astype(np.float32)
+    W, b = net.unpack()
+    M.ACT = "gelu_poly"
+    try:
+        loss, g = net.grad(X, T, mode=0)
+        l_ref, gW, gb = M.loss_and_grads([w.astype(np.float64) for w in W], [x.astype(np.float64) for x in b],
+                                         X.astype(np.float64), T.astype(np.float64),
+                                         *[x.astype(np.float64) for x in nm], mode="fp64")
+    finally:
+        M.ACT = "relu"
+    gr = flat(gW, gb)
+    print(f"n {n}: loss {abs(loss - l_ref) / l_ref:.1e}, gradient {np.linalg.norm(g - gr) / np.linalg.norm(gr):.1e}",
+          flush=True)
+    assert abs(loss - l_ref) < 1e-5 * l_ref
+    assert np.linalg.norm(g - gr) < 1e-5 * np.linalg.norm(gr)
+    net.close()
