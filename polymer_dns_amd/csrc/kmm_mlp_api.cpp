@@ -3,6 +3,7 @@
 // mini-batches.  No reference counterpart (the network is new).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -172,6 +173,18 @@ extern "C" int kmm_mlp_grad(kmm_mlp* n, int npts, const float* X, const float* T
   return KMM_OK;
 }
 
+// the two sample blocks of a training call: their events, and the wait for
+// everything queued before the host blocks go away (also on an error)
+struct TrainSync {
+  hipStream_t s;
+  hipEvent_t done[2] = {nullptr, nullptr};
+  ~TrainSync() {
+    hipStreamSynchronize(s);
+    for (hipEvent_t e : done)
+      if (e) hipEventDestroy(e);
+  }
+};
+
 // Adam training on (X, T): `steps` mini-batches of `batch` samples drawn
 // without replacement from a seeded permutation (reshuffled every epoch);
 // losses[s] (may be NULL) receives the batch loss before update s.
@@ -180,35 +193,56 @@ extern "C" int kmm_mlp_train(kmm_mlp* n, int npts, const float* X, const float* 
   if (!n || npts <= 0 || !X || !T || steps < 0 || batch <= 0 || batch > npts || !(lr > 0.0f))
     return mfail(KMM_E_ARG, "bad argument");
   MHIP(hipSetDevice(n->device));
-  // batches are copied in order from a host-side shuffled copy
+  // Batches are drawn in order from a host-side shuffled index.  The samples
+  // of several steps (at most 4 MB) are gathered into one host block, copied
+  // at once and trained on without waiting; two blocks alternate, so that
+  // the next one is gathered while the GPU trains on this one.  (A copy and
+  // a wait per step took 0.098 ms a step at 1024 samples, this 0.067, of
+  // which the GPU's work is 0.057.)
   std::vector<int> perm(npts);
   std::iota(perm.begin(), perm.end(), 0);
   std::mt19937_64 rng(seed);
-  std::vector<float> bx((size_t)batch * 22), bt((size_t)batch * 6);
+  const size_t bs = (size_t)batch * 28;   // floats of a batch: X, then T
+  const int S = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::max(steps, 1), ((size_t)1 << 20) / bs));
+  std::vector<float> host[2];
   int r;
-  if ((r = grow(&n->X, &n->capX, (size_t)batch * 22)) || (r = grow(&n->T, &n->capT, (size_t)batch * 6)) ||
-      (r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(batch))))
+  if ((r = grow(&n->X, &n->capX, 2 * S * bs)) || (r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(batch))) ||
+      (losses && (r = grow(&n->T, &n->capT, (size_t)steps))))
     return r;
+  TrainSync sync{n->stream};
   int pos = npts;
-  for (int s = 0; s < steps; ++s) {
-    if (pos + batch > npts) {
-      std::shuffle(perm.begin(), perm.end(), rng);
-      pos = 0;
+  for (int s0 = 0, b = 0; s0 < steps; s0 += S, b ^= 1) {
+    const int ns = std::min(S, steps - s0);
+    if (sync.done[b]) MHIP(hipEventSynchronize(sync.done[b]));  // the block's last copy and steps have ended
+    host[b].resize((size_t)S * bs);
+    for (int s = 0; s < ns; ++s) {
+      if (pos + batch > npts) {
+        std::shuffle(perm.begin(), perm.end(), rng);
+        pos = 0;
+      }
+      float* bx = host[b].data() + (size_t)s * bs;
+      float* bt = bx + (size_t)batch * 22;
+      for (int i = 0; i < batch; ++i) {
+        const int q = perm[pos + i];
+        std::memcpy(bx + (size_t)i * 22, X + (size_t)q * 22, 22 * sizeof(float));
+        std::memcpy(bt + (size_t)i * 6, T + (size_t)q * 6, 6 * sizeof(float));
+      }
+      pos += batch;
     }
-    for (int i = 0; i < batch; ++i) {
-      const int q = perm[pos + i];
-      std::memcpy(&bx[(size_t)i * 22], X + (size_t)q * 22, 22 * sizeof(float));
-      std::memcpy(&bt[(size_t)i * 6], T + (size_t)q * 6, 6 * sizeof(float));
+    float* dx = n->X + (size_t)b * S * bs;
+    MHIP(hipMemcpyAsync(dx, host[b].data(), (size_t)ns * bs * sizeof(float), hipMemcpyHostToDevice, n->stream));
+    for (int s = 0; s < ns; ++s) {
+      const float* x = dx + (size_t)s * bs;
+      MHIP(kmm::launch_mlp_train_step(batch, x, x + (size_t)batch * 22, n->par, n->norm, 1 | (n->act << 1), n->ws, n->g,
+                                      losses ? n->T + s0 + s : n->loss, n->m, n->v, lr, ++n->adam_t, n->wb,
+                                      n->stream));
     }
-    pos += batch;
-    MHIP(hipMemcpyAsync(n->X, bx.data(), bx.size() * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    MHIP(hipMemcpyAsync(n->T, bt.data(), bt.size() * sizeof(float), hipMemcpyHostToDevice, n->stream));
-    MHIP(kmm::launch_mlp_train_step(batch, n->X, n->T, n->par, n->norm, 1 | (n->act << 1), n->ws, n->g, n->loss, n->m,
-                                    n->v, lr, ++n->adam_t, n->wb, n->stream));
-    if (losses) MHIP(hipMemcpyAsync(losses + s, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream));
-    // the host buffers are reused by the next batch
-    MHIP(hipStreamSynchronize(n->stream));
+    if (!sync.done[b]) MHIP(hipEventCreateWithFlags(&sync.done[b], hipEventDisableTiming));
+    MHIP(hipEventRecord(sync.done[b], n->stream));
   }
+  if (losses && steps > 0)
+    MHIP(hipMemcpyAsync(losses, n->T, (size_t)steps * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+  MHIP(hipStreamSynchronize(n->stream));
   return KMM_OK;
 }
 
