@@ -61,6 +61,7 @@ struct kmm_ctx {
   size_t vsz = 16;         // bytes per complex transfer element (16 FP64, 8 mixed)
   double *smz, *smy, *seght_d;
   unsigned long long* cfl_d;
+  double* cflpart = nullptr;  // [nyp mz / 8] block maxima of the evaluation in flight
   int cfl_cap = 0;
   // immersed boundary
   int nsrc = 0;
@@ -397,6 +398,7 @@ static PlaneArgs plane_args(kmm_ctx* c, int it, unsigned long long* cfl) {
   a.Z = c->Z; a.ZF = c->ZF;
   for (int o = 0; o < 4; ++o) a.out[o] = c->NL[o];
   a.cfl = cfl;
+  a.cflpart = c->cflpart; a.ncfl = c->nyp * (c->mz / 8);
   a.nsrc = c->nsrc; a.src = c->src; a.srcp = c->srcp; a.fint = c->fint; a.drag = c->drag;
   a.gain = c->cfg.gain; a.ugain = c->cfg.ugain; a.it = it; a.perturbtime = c->cfg.perturbtime;
   a.trow = c->trow; a.tx = c->tx; a.tptr = c->tptr; a.ent_src = c->ent_src; a.ent_w = c->ent_w;
@@ -493,6 +495,7 @@ extern "C" int kmm_create(const kmm_config* cfg, int device, kmm_ctx** out) {
       if ((r = dalloc(c, (void**)&c->scsrc, (size_t)c->nyp * c->mz * c->mx * sizeof(double)))) goto fail_;
     if ((r = dalloc(c, (void**)&c->cfl_d, 4096 * sizeof(unsigned long long)))) goto fail_;
     c->cfl_cap = 4096;
+    if ((r = dalloc(c, (void**)&c->cflpart, (size_t)c->nyp * (c->mz / 8) * sizeof(double)))) goto fail_;
     // twiddles and smoothing
     auto up = [&](void** d, const void* h, size_t b) -> int {
       int rr = dalloc(c, d, b);

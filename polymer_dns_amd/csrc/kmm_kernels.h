@@ -114,6 +114,8 @@ struct PlaneArgs {
   void* ZF;            // [nfout][nyp][mz][nxh]
   void* out[4];        // NL [y][kx][kz]
   unsigned long long* cfl;  // bit pattern of the max CFL number for this call
+  double* cflpart;     // [ncfl] block maxima of k_xplane (ncfl = nyp mz / 8 blocks; 0: no CFL number)
+  int ncfl;
   // immersed boundary (Goldstein feedback, solvers.f90:2996-3108)
   int nsrc;
   const int4* src;        // (y, z, x, imatrix type) per solid cell

@@ -328,8 +328,20 @@ __device__ __forceinline__ void xplane_body(const PlaneArgs& A, int bid) {
       else    { ph[0][m].x = o0; ph[1][m].x = o1; ph[2][m].x = o2; if (NFOUT == 4) ph[3][m].x = vc; }
     }
   }
+  // the block's largest CFL number: k_zfwd's last block takes the maximum
+  // over the blocks.  (An atomicMax per wave on one address ran at one per
+  // 13 ns whatever the field's precision, 160 of the 165 to 192 us of this
+  // kernel at 128 x 129 x 128: 12 384 waves.)
+  __shared__ double cw[WPB];
   cmax = wave_max(cmax);
-  if (lane == 0) atomicMax(A.cfl, (unsigned long long)__double_as_longlong(cmax));
+  if (lane == 0) cw[wv] = cmax;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double b = cw[0];
+#pragma unroll
+    for (int w = 1; w < WPB; ++w) b = fmax(b, cw[w]);
+    A.cflpart[bid] = b;
+  }
   if (A.nsrc > 0) {
     // gathered spreading of the feedback force onto targets of rows zA, zB;
     // the lane owning x adds (x = lane + 64 m)
@@ -422,7 +434,24 @@ __device__ __forceinline__ void zfwd_tile_load(T (&px)[TL], T (&py)[TL], const V
   }
 }
 
-// Work items (output field, y, group of 8 kx lines) walked like k_zinv's.
+// the step's CFL number from the block maxima of k_xplane, by one block
+__device__ __forceinline__ void cfl_reduce(const PlaneArgs& A) {
+  __shared__ double cw[8];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double c = 0.0;
+  for (int e = threadIdx.x; e < A.ncfl; e += 512) c = fmax(c, A.cflpart[e]);
+  c = wave_max(c);
+  if (lane == 0) cw[wv] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 8; ++w) c = fmax(c, cw[w]);
+    *A.cfl = (unsigned long long)__double_as_longlong(c);
+  }
+}
+
+// Work items (output field, y, group of 8 kx lines) walked like k_zinv's;
+// with ncfl > 0 one more block than the items need forms the CFL number.
 template <int MZ, int NFOUT, typename V>
 __device__ __forceinline__ void zfwd_body(const PlaneArgs& A, int bid) {
   using T = typename Scal<V>::T;
@@ -432,6 +461,11 @@ __device__ __forceinline__ void zfwd_body(const PlaneArgs& A, int bid) {
   const int ngx = A.nxh / 8;
   const int ngroups = A.nyp * ngx;
   const int nitems = NFOUT * ngroups;
+  const int nwalk = (int)gridDim.x - (A.ncfl > 0 ? 1 : 0);  // blocks that walk the items
+  if (bid == nwalk) {
+    cfl_reduce(A);
+    return;
+  }
   constexpr int BL = FFTBuf<MZ>::len;
   V* buf = sm + wv * BL;
   V* scr = buf;  // in place
@@ -458,7 +492,7 @@ __device__ __forceinline__ void zfwd_body(const PlaneArgs& A, int bid) {
     const V* sp = src(it, k0);
     zfwd_tile_load<MZ, TL, V, T>(prx, pry, sp, A.nxh, k0);
   }
-  for (; it < nitems; it += gridDim.x) {
+  for (; it < nitems; it += nwalk) {
     const int o = it / ngroups, g = it - o * ngroups;
     const int y = g / ngx, kx0 = (g - y * ngx) * 8;
     const int kx = kx0 + wv;
@@ -470,9 +504,9 @@ __device__ __forceinline__ void zfwd_body(const PlaneArgs& A, int bid) {
       if (e < MZ * 8) sm[(e & 7) * BL + fpad(e >> 3)] = mkv<V>(prx[q], pry[q]);
     }
     __syncthreads();
-    if (it + (int)gridDim.x < nitems) {
+    if (it + nwalk < nitems) {
       int k0;
-      const V* sp = src(it + gridDim.x, k0);
+      const V* sp = src(it + nwalk, k0);
       zfwd_tile_load<MZ, TL, V, T>(prx, pry, sp, A.nxh, k0);
     }
     const V* r = wave_fft<MZ, -1, V, kPlanePlan>(buf, scr, tw, lane);
@@ -537,7 +571,7 @@ static void launch_zfwd(const PlaneArgs& a, hipStream_t s) {
   const int nitems = NFOUT * a.nyp * (a.nxh / 8);
   static ZGridCache cache;
   const int grid = zitems_grid(cache, k_zfwd<MZ, NFOUT, V>, zlds, nitems);
-  hipLaunchKernelGGL((k_zfwd<MZ, NFOUT, V>), dim3(grid), dim3(512), zlds, s, a);
+  hipLaunchKernelGGL((k_zfwd<MZ, NFOUT, V>), dim3(grid + (a.ncfl > 0 ? 1 : 0)), dim3(512), zlds, s, a);
 }
 
 // ------------------------------------------------------------ launchers --
@@ -1151,7 +1185,7 @@ static hipError_t plane_batch_impl(const PlaneArgs& a, const PlaneArgs* dA, int 
     static ZGridCache cache;
     const int cap = zitems_grid(cache, k_zfwd_batch<MZ, NFOUT, V>, zlds, 1 << 30);
     const int grid = std::min(nitems, std::max(1, (cap + nmem - 1) / nmem));
-    hipLaunchKernelGGL((k_zfwd_batch<MZ, NFOUT, V>), dim3(grid, nmem), dim3(512), zlds, s, dA);
+    hipLaunchKernelGGL((k_zfwd_batch<MZ, NFOUT, V>), dim3(grid + (a.ncfl > 0 ? 1 : 0), nmem), dim3(512), zlds, s, dA);
   }
   return hipGetLastError();
 }
