@@ -18,13 +18,14 @@
 
 #include "kmm_kernels.h"
 #include "kmm_device.h"
+#include "kmm_xfft.h"
 
 namespace kmm {
 
-// FFT plan cost model of the x and z transforms (make_plan): 1, fewest
-// vector instructions per lane.  Measured against fewest rounds at 128^3
-// FP64: k_zinv -11 %, k_zfwd -9 %, k_xplane -3 % (more LDS passes, fewer
-// idle lanes in the radix-8 stages).
+// FFT plan cost model of the z transforms (make_plan): 1, fewest vector
+// instructions per lane.  Measured against fewest rounds at 128^3 FP64:
+// k_zinv -11 %, k_zfwd -9 % (more LDS passes, fewer idle lanes in the radix-8
+// stages).
 constexpr int kPlanePlan = 1;
 
 // one wave's line of nz spectral values, NJ per lane
@@ -195,95 +196,97 @@ __global__ __launch_bounds__(256) void k_ibdrag(PlaneArgs A) {
   }
 }
 
-// the two z rows (A, B) of one field, nxh spectral values each, NK per lane
-template <int NK, typename V, typename T>
-__device__ __forceinline__ void xrow_pair_load(T (&ax)[NK], T (&ay)[NK], T (&bx)[NK], T (&by)[NK],
-                                               const V* __restrict__ ra, const V* __restrict__ rb, int nxh,
-                                               int lane) {
-#pragma unroll
-  for (int q = 0; q < NK; ++q) {
-    const int k = min(lane + 64 * q, nxh - 1);  // in range; lanes past nxh do not use theirs
-    const V a = ra[k], b = rb[k];
-    ax[q] = a.x; ay[q] = a.y; bx[q] = b.x; by[q] = b.y;
-  }
+// field of the f-th line of k_xplane: with a scalar, its gradient right after
+// the velocity
+template <int NFIN>
+__host__ __device__ constexpr int xfield(int f) { return NFIN == 9 && f >= 3 ? (f < 6 ? f + 3 : f - 3) : f; }
+// lines per wavefront of k_xplane (its inverse and forward batches)
+template <int MX, int NFIN, int NFOUT>
+constexpr int xplane_lines() {
+  const int a = xlines<MX, NFIN>(), b = xlines<MX, NFOUT>();
+  return a > b ? a : b;
 }
 
-// TV: occupancy variant picked by the autotuner (0: the compiler's register
-// budget; 1: one more wave per SIMD than FP64/FP32 need at MX = 192, i.e.
-// >= 3 (FP64) or >= 5 (FP32) waves/SIMD)
+// A wavefront holds one pair of z rows: each field's two real rows are one
+// complex x line, transformed NB lines at a time (kmm_xfft.h); the points
+// x = lane + 64 m of all fields stay in registers for the products.
+// TV: occupancy variant picked by the autotuner (0: two waves per SIMD in
+// FP64, the compiler's choice in FP32; 1: three and five.  At 128 x 129 x 128
+// with the scalar FP64 0.135 / 0.146 ms, FP32 0.072 / 0.072 ms)
 template <int MX, int NFIN, int NFOUT, int WPB, typename V>
 __device__ __forceinline__ void xplane_body(const PlaneArgs& A, int bid) {
   using T = typename Scal<V>::T;
+  using XF = XFft<MX>;
   constexpr int XPL = (MX + 63) / 64;  // x positions per lane: x = lane + 64 m
+  constexpr int nxh = MX / 3;
   extern __shared__ __align__(16) unsigned char smraw[];
   V* sm = reinterpret_cast<V*>(smraw);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int nzb = A.mz / (2 * WPB);
   const int y = bid / nzb;
   const int zA = (bid % nzb) * 2 * WPB + 2 * wv, zB = zA + 1;
-  constexpr int BL = FFTBuf<MX>::len;
   V* tw = sm;                              // [MX] twiddles
-  V* buf = sm + MX + (size_t)wv * 2 * BL;
-  V* scr = buf + BL;
+  constexpr int NI = xlines<MX, NFIN>(), NC = (NFIN + NI - 1) / NI;  // inverse: lines a batch, batches
+  constexpr int NO = xlines<MX, NFOUT>();                        // forward: lines a batch
+  V* buf = sm + MX + (size_t)wv * xplane_lines<MX, NFIN, NFOUT>() * XF::BUF;
   for (int e = threadIdx.x; e < MX; e += WPB * 64) tw[e] = static_cast<const V*>(A.twX)[e];
   __syncthreads();
-  const int nxh = A.nxh;
   // ph[f][m] = (row A, row B) physical values at x = lane + 64 m
   V ph[NFIN][XPL];
-  // the next field's two rows are loaded into registers during this field's
-  // transform (nxh = MX/3 values per row)
   constexpr int NK = (MX / 3 + 63) / 64;
-  T pax[NK], pay[NK], pbx[NK], pby[NK];
-  auto rows = [&](int f) {
-    const V* zr = static_cast<const V*>(A.Z) + ((size_t)f * A.nyp + y) * A.mz * nxh;
-    xrow_pair_load<NK, V, T>(pax, pay, pbx, pby, zr + (size_t)zA * nxh, zr + (size_t)zB * nxh, nxh, lane);
+  constexpr bool XPRE = !(sizeof(V) == 16 && MX > 288);  // FP64 at 384: no registers for it
+  V pa[NI][NK], pb[NI][NK];  // the next batch's rows, loaded during this one's transforms
+  auto rows = [&](int f0) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (f0 + i >= NFIN) continue;
+      const V* ra = static_cast<const V*>(A.Z) + (((size_t)xfield<NFIN>(f0 + i) * A.nyp + y) * A.mz + zA) * nxh;
+#pragma unroll
+      for (int q = 0; q < NK; ++q) {
+        const int k = min(lane + 64 * q, nxh - 1);  // in range; lanes past nxh do not use theirs
+        pa[i][q] = ra[k];
+        pb[i][q] = ra[nxh + k];
+      }
+    }
+  };
+  // -u.grad(theta) + source into ph[6] once its six fields are there: the
+  // scalar's gradient does not stay in registers (the empty asm keeps the
+  // compiler from forming it later)
+  const T src_u = (T)A.src_uniform;
+  auto scalar_terms = [&]() {
+#pragma unroll
+    for (int m = 0; m < XPL; ++m) {
+      const bool ok = (lane + 64 * m) < MX;
+#pragma unroll
+      for (int rr = 0; rr < 2; ++rr) {
+        const T u = rr ? ph[0][m].y : ph[0][m].x, v = rr ? ph[1][m].y : ph[1][m].x;
+        const T w = rr ? ph[2][m].y : ph[2][m].x, tx = rr ? ph[6][m].y : ph[6][m].x;
+        const T ty = rr ? ph[7][m].y : ph[7][m].x, tz = rr ? ph[8][m].y : ph[8][m].x;
+        T vc = -(u * tx + v * ty + w * tz) + src_u;
+        if (A.scsrc && ok)  // vc += scsource/dt (solvers.f90:3061-3063)
+          vc += (T)(A.scsrc[((size_t)y * A.mz + (rr ? zB : zA)) * MX + lane + 64 * m] / A.dt);
+        asm volatile("" : "+v"(vc));
+        if (rr) ph[6][m].y = vc; else ph[6][m].x = vc;
+      }
+    }
   };
   rows(0);
-  // MX = 64 R with R the plan's last radix: the last stage of an inverse
-  // transform leaves lane j the outputs x = j + 64 m, which can stay in
-  // registers, and a forward transform can run the reversed plan, whose
-  // first stage reads them there.  Measured at MX = 192: FP32 gains from the
-  // inverse side (the forward side costs registers), FP64 from the forward
-  // side (the inverse side takes it from 3 to 2 waves per SIMD).
-  constexpr bool XOK = MX % 64 == 0 && plan_last_radix<MX, kPlanePlan>() == MX / 64;
-  constexpr bool XINV = XOK && sizeof(V) == 8, XFWD = XOK && sizeof(V) == 16;
-  // FP64: twiddles as powers of one table value per butterfly (fewer LDS
-  // loads in this LDS-bound kernel, -3 % at MX = 192; no gain in FP32)
-  constexpr bool XTW = sizeof(V) == 16;
-  const V none[8] = {};
-  V regs[8];
 #pragma unroll
-  for (int f = 0; f < NFIN; ++f) {
-    // zeros at the dealiasing band [nxh, MX - nxh]; the packed rows fill the rest
-    for (int x = nxh + lane; x <= MX - nxh; x += 64) buf[fpad(x)] = vzero<V>();
+  for (int c = 0; c < NC; ++c) {
+    const int f0 = c * NI;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (f0 + i < NFIN) xline_pack<MX, V>(buf, i, pa[i], pb[i], lane);
+    if (XPRE && c + 1 < NC) rows(f0 + NI);
+    xfft_inv<MX, NI, V>(buf, tw, lane);
+    if (!XPRE && c + 1 < NC) rows(f0 + NI);
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (f0 + i < NFIN) xline_read<MX, V>(buf, i, ph[xfield<NFIN>(f0 + i)], lane);
     wave_sync();
-#pragma unroll
-    for (int q = 0; q < NK; ++q) {
-      const int k = lane + 64 * q;
-      if (k >= nxh) continue;
-      const V ua = mkv<V>(pax[q], pay[q]), ub = mkv<V>(pbx[q], pby[q]);
-      if (k == 0) {
-        buf[0] = mkv<V>(ua.x, ub.x);
-      } else {
-        buf[fpad(k)] = mkv<V>(ua.x - ub.y, ua.y + ub.x);
-        buf[fpad(MX - k)] = mkv<V>(ua.x + ub.y, ub.x - ua.y);
-      }
+    if constexpr (NFIN == 9) {
+      if (f0 < 6 && f0 + NI >= 6) scalar_terms();
     }
-    if (f + 1 < NFIN) rows(f + 1);
-    wave_sync();
-    if constexpr (XINV) {
-      wave_fft_ex<MX, +1, V, kPlanePlan, false, false, true, XTW>(buf, scr, tw, lane, none, regs);
-#pragma unroll
-      for (int m = 0; m < XPL; ++m) ph[f][m] = regs[m];
-    } else {
-      V* r = wave_fft_ex<MX, +1, V, kPlanePlan, false, false, false, XTW>(buf, scr, tw, lane, none, regs);
-#pragma unroll
-      for (int m = 0; m < XPL; ++m) {
-        const int x = lane + 64 * m;
-        ph[f][m] = (x < MX) ? r[fpad(x)] : vzero<V>();
-      }
-    }
-    wave_sync();
   }
   // physical u, v, w for particle tracking (up3d/vp3d/wp3d, solvers.f90:3113-3115)
   if (A.cap) {
@@ -301,9 +304,8 @@ __device__ __forceinline__ void xplane_body(const PlaneArgs& A, int bid) {
     }
   }
   // pointwise products (solvers.f90:2891-2898), CFL (2985-2986), dPdx (3044)
-  const T sgy = (T)A.seght[y];
   const T dpdx = (T)((A.flow_select == 1) ? (A.dpdx_d ? *A.dpdx_d : A.dPdx) : 0.0);
-  const T delxm = (T)A.delxm, delzm = (T)A.delzm, dt = (T)A.dt, src_u = (T)A.src_uniform;
+  const T cx = (T)(A.dt / A.delxm), cy = (T)(A.dt / A.seght[y]), cz = (T)(A.dt / A.delzm);
   double cmax = 0.0;
 #pragma unroll
   for (int m = 0; m < XPL; ++m) {
@@ -313,15 +315,8 @@ __device__ __forceinline__ void xplane_body(const PlaneArgs& A, int bid) {
       const T u = rr ? ph[0][m].y : ph[0][m].x, v = rr ? ph[1][m].y : ph[1][m].x;
       const T w = rr ? ph[2][m].y : ph[2][m].x, ox = rr ? ph[3][m].y : ph[3][m].x;
       const T oy = rr ? ph[4][m].y : ph[4][m].x, oz = rr ? ph[5][m].y : ph[5][m].x;
-      T vc = 0;
-      if (NFIN == 9) {
-        const T tx = rr ? ph[6][m].y : ph[6][m].x, ty = rr ? ph[7][m].y : ph[7][m].x;
-        const T tz = rr ? ph[8][m].y : ph[8][m].x;
-        vc = -(u * tx + v * ty + w * tz) + src_u;
-        if (A.scsrc && ok)  // vc += scsource/dt (solvers.f90:3061-3063)
-          vc += (T)(A.scsrc[((size_t)y * A.mz + (rr ? zB : zA)) * MX + lane + 64 * m] / A.dt);
-      }
-      const double c = (double)((fabs(u) / delxm + fabs(v) / sgy + fabs(w) / delzm) * dt);
+      const T vc = NFOUT == 4 ? (rr ? ph[NFIN == 9 ? 6 : 0][m].y : ph[NFIN == 9 ? 6 : 0][m].x) : (T)0;
+      const double c = (double)(fabs(u) * cx + fabs(v) * cy + fabs(w) * cz);
       if (ok) cmax = fmax(cmax, c);
       const T o0 = v * oz - w * oy - dpdx, o1 = -u * oz + w * ox, o2 = u * oy - v * ox;
       if (rr) { ph[0][m].y = o0; ph[1][m].y = o1; ph[2][m].y = o2; if (NFOUT == 4) ph[3][m].y = vc; }
@@ -382,40 +377,28 @@ __device__ __forceinline__ void xplane_body(const PlaneArgs& A, int bid) {
   }
   // forward x transforms (r2c) of the outputs, two rows per transform
 #pragma unroll
-  for (int o = 0; o < NFOUT; ++o) {
-    V* r;
-    if constexpr (XFWD) {
+  for (int o0 = 0; o0 < NFOUT; o0 += NO) {
 #pragma unroll
-      for (int m = 0; m < XPL; ++m) regs[m] = ph[o][m];
-      r = wave_fft_ex<MX, -1, V, kPlanePlan, true, true, false, XTW>(buf, scr, tw, lane, regs, regs);
-    } else {
+    for (int i = 0; i < NO; ++i)
+      if (o0 + i < NFOUT) xline_write<MX, V>(buf, i, ph[o0 + i], lane);
+    xfft_fwd<MX, NO, V>(buf, tw, lane);
 #pragma unroll
-      for (int m = 0; m < XPL; ++m) {
-        const int x = lane + 64 * m;
-        if (x < MX) buf[fpad(x)] = ph[o][m];
-      }
-      wave_sync();
-      r = wave_fft_ex<MX, -1, V, kPlanePlan, false, false, false, XTW>(buf, scr, tw, lane, none, regs);
-    }
-    V* zo = static_cast<V*>(A.ZF) + ((size_t)o * A.nyp + y) * A.mz * nxh;
-    for (int k = lane; k < nxh; k += 64) {
-      const V zk = r[fpad(k)], zm = r[fpad((MX - k) % MX)];
-      const V ua = mkv<V>((T)0.5 * (zk.x + zm.x), (T)0.5 * (zk.y - zm.y));
-      const V ub = mkv<V>((T)0.5 * (zk.y + zm.y), (T)-0.5 * (zk.x - zm.x));
-      zo[(size_t)zA * nxh + k] = ua;
-      zo[(size_t)zB * nxh + k] = ub;
+    for (int i = 0; i < NO; ++i) {
+      if (o0 + i >= NFOUT) continue;
+      V* zo = static_cast<V*>(A.ZF) + (((size_t)(o0 + i) * A.nyp + y) * A.mz + zA) * nxh;
+      xline_unpack<MX, V>(buf, i, zo, zo + nxh, lane);
     }
     wave_sync();
   }
 }
 
 template <int MX, int NFIN, int NFOUT, int WPB, typename V, int TV = 0>
-__global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(TV ? (sizeof(V) == 16 ? 3 : 5) : 1)))
+__global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(TV ? (sizeof(V) == 16 ? 3 : 5) : (sizeof(V) == 16 ? 2 : 1))))
 void k_xplane(PlaneArgs A) {
   xplane_body<MX, NFIN, NFOUT, WPB, V>(A, blockIdx.x);
 }
 template <int MX, int NFIN, int NFOUT, int WPB, typename V, int TV = 0>
-__global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(TV ? (sizeof(V) == 16 ? 3 : 5) : 1)))
+__global__ __launch_bounds__(WPB * 64) __attribute__((amdgpu_waves_per_eu(TV ? (sizeof(V) == 16 ? 3 : 5) : (sizeof(V) == 16 ? 2 : 1))))
 void k_xplane_batch(const PlaneArgs* __restrict__ AA) {
   xplane_body<MX, NFIN, NFOUT, WPB, V>(AA[blockIdx.y], blockIdx.x);
 }
@@ -580,35 +563,11 @@ static void launch_zfwd(const PlaneArgs& a, hipStream_t s) {
 // complex x transform: spectra a_k, b_k (k < nxh) of the two fields are
 // packed as a + i b with the Hermitian extension; after the inverse
 // transform the real part is field a, the imaginary part field b.  With
-// dxa/dxb the spectrum is first multiplied by i alpha k (d/dx).
-// forward r2c of two real rows through one complex transform; writes the
-// nxh kept modes of each (the 1/(mx mz) scale is applied in k_zfwd)
-template <int MX, typename V>
-__device__ __forceinline__ void xrow_pair_fwd(const typename Scal<V>::T (&a)[(MX + 63) / 64],
-                                              const typename Scal<V>::T (&b)[(MX + 63) / 64], V* __restrict__ oa,
-                                              V* __restrict__ ob, int nxh, V* buf, V* scr, const V* tw, int lane) {
-  using T = typename Scal<V>::T;
-  constexpr int XPL = (MX + 63) / 64;
-#pragma unroll
-  for (int m = 0; m < XPL; ++m) {
-    const int x = lane + 64 * m;
-    if (x < MX) buf[fpad(x)] = mkv<V>(a[m], b[m]);
-  }
-  wave_sync();
-  // FP64: twiddles as powers of one table value per butterfly (fewer LDS loads)
-  const V none[8] = {};
-  V unused[8];
-  V* r = wave_fft_ex<MX, -1, V, kPlanePlan, false, false, false, sizeof(V) == 16>(buf, scr, tw, lane, none, unused);
-  for (int k = lane; k < nxh; k += 64) {
-    const V zk = r[fpad(k)], zm = r[fpad((MX - k) % MX)];
-    oa[k] = mkv<V>((T)0.5 * (zk.x + zm.x), (T)0.5 * (zk.y - zm.y));
-    ob[k] = mkv<V>((T)0.5 * (zk.y + zm.y), (T)-0.5 * (zk.x - zm.x));
-  }
-  wave_sync();
-}
-
+// dxa/dxb the spectrum is first multiplied by i alpha k (d/dx).  NB pairs
+// are transformed at a time (kmm_xfft.h).
+//
 // Spectral inputs of one pair transform, kept in registers so that the
-// loads of the next pair overlap the current transform.
+// loads of the next pairs overlap the current transforms.
 template <int MX, typename V>
 struct PairIn {
   static constexpr int KPL = (MX / 3 + 63) / 64;  // nxh = MX/3 modes over 64 lanes
@@ -616,53 +575,42 @@ struct PairIn {
 };
 template <int MX, typename V>
 __device__ __forceinline__ void pair_load(PairIn<MX, V>& r, const V* __restrict__ ra, const V* __restrict__ rb,
-                                          int nxh, int lane) {
+                                          int lane) {
 #pragma unroll
   for (int j = 0; j < PairIn<MX, V>::KPL; ++j) {
-    const int k = lane + 64 * j;
-    if (k < nxh) {
-      r.a[j] = ra[k];
-      r.b[j] = rb[k];
-    }
+    const int k = min(lane + 64 * j, MX / 3 - 1);  // in range; lanes past nxh do not use theirs
+    r.a[j] = ra[k];
+    r.b[j] = rb[k];
   }
 }
 template <int MX, typename V>
-__device__ __forceinline__ void pair_inv(const PairIn<MX, V>& r, bool dxa, bool dxb, int nxh, double alpha, V* buf,
-                                         V* scr, const V* tw, int lane, typename Scal<V>::T (&oa)[(MX + 63) / 64],
-                                         typename Scal<V>::T (&ob)[(MX + 63) / 64]) {
+__device__ __forceinline__ void pair_pack(const PairIn<MX, V>& r, bool dxa, bool dxb, double alpha, V* buf, int g,
+                                          int lane) {
   using T = typename Scal<V>::T;
-  constexpr int XPL = (MX + 63) / 64;
-  // zeros at the dealiasing band [nxh, MX - nxh]; the packed spectra fill the rest
-  for (int x = nxh + lane; x <= MX - nxh; x += 64) buf[fpad(x)] = vzero<V>();
-  wave_sync();
+  PairIn<MX, V> u = r;
 #pragma unroll
   for (int j = 0; j < PairIn<MX, V>::KPL; ++j) {
-    const int k = lane + 64 * j;
-    if (k < nxh) {
-      V ua = r.a[j], ub = r.b[j];
-      const T wk = (T)(alpha * (double)k);
-      if (dxa) ua = mkv<V>(-ua.y * wk, ua.x * wk);
-      if (dxb) ub = mkv<V>(-ub.y * wk, ub.x * wk);
-      if (k == 0) {
-        buf[0] = mkv<V>(ua.x, ub.x);
-      } else {
-        buf[fpad(k)] = mkv<V>(ua.x - ub.y, ua.y + ub.x);
-        buf[fpad(MX - k)] = mkv<V>(ua.x + ub.y, ub.x - ua.y);
-      }
-    }
+    const T wk = (T)(alpha * (double)(lane + 64 * j));
+    if (dxa) u.a[j] = mkv<V>(-u.a[j].y * wk, u.a[j].x * wk);
+    if (dxb) u.b[j] = mkv<V>(-u.b[j].y * wk, u.b[j].x * wk);
   }
-  wave_sync();
-  const V none[8] = {};
-  V unused[8];
-  V* res = wave_fft_ex<MX, +1, V, kPlanePlan, false, false, false, sizeof(V) == 16>(buf, scr, tw, lane, none, unused);
+  xline_pack<MX, V>(buf, g, u.a, u.b, lane);
+}
+template <int MX, typename V>
+__device__ __forceinline__ void pair_read(const V* buf, int g, typename Scal<V>::T (&oa)[(MX + 63) / 64],
+                                          typename Scal<V>::T (&ob)[(MX + 63) / 64], int lane) {
+  V p[(MX + 63) / 64];
+  xline_read<MX, V>(buf, g, p, lane);
 #pragma unroll
-  for (int m = 0; m < XPL; ++m) {
-    const int x = lane + 64 * m;
-    const V v = (x < MX) ? res[fpad(x)] : vzero<V>();
-    oa[m] = v.x;
-    ob[m] = v.y;
-  }
-  wave_sync();
+  for (int m = 0; m < (MX + 63) / 64; ++m) { oa[m] = p[m].x; ob[m] = p[m].y; }
+}
+template <int MX, typename V>
+__device__ __forceinline__ void pair_write(V* buf, int g, const typename Scal<V>::T (&a)[(MX + 63) / 64],
+                                           const typename Scal<V>::T (&b)[(MX + 63) / 64], int lane) {
+  V p[(MX + 63) / 64];
+#pragma unroll
+  for (int m = 0; m < (MX + 63) / 64; ++m) p[m] = mkv<V>(a[m], b[m]);
+  xline_write<MX, V>(buf, g, p, lane);
 }
 
 // The 18 pair transforms of a row: field ids >= 0 index the z-stage outputs
@@ -715,16 +663,17 @@ template <int MX, typename V>
 struct PolyRow {
   using T = typename Scal<V>::T;
   static constexpr int XPL = (MX + 63) / 64;
+  static constexpr int PB = xlines<MX, 3>();  // pairs per batch (divides 18)
   T u[3][XPL], c[XPL][6], s[XPL][6];
-  PairIn<MX, V> pin[2];
+  PairIn<MX, V> pin[PB];
   const V* U;
   const V* ZP;
   V* ZF;
   size_t plane, roff;
-  int nxh, lane, ipeter;
+  int lane, ipeter;
   double alpha;
   T L2;
-  V *buf, *scr;
+  V* buf;
   const V* tw;
   float* capg;   // nullptr or [9][P] physical du_i/dx_k (FP32)
   float* caps;   // nullptr or [6][P] physical Peterlin stress (FP32)
@@ -741,20 +690,50 @@ struct PolyRow {
     }
   }
 
+  // load the pairs of batch C
+  template <int C, int I = 0>
+  __device__ __forceinline__ void load() {
+    if constexpr (I < PB && C * PB + I < kNP) {
+      constexpr PairSpec sp = poly_pair(C * PB + I);
+      pair_load<MX, V>(pin[I], rowp(sp.fa), rowp(sp.fb), lane);
+      load<C, I + 1>();
+    }
+  }
+  template <int C, int I = 0>
+  __device__ __forceinline__ void pack() {
+    if constexpr (I < PB && C * PB + I < kNP) {
+      constexpr PairSpec sp = poly_pair(C * PB + I);
+      pair_pack<MX, V>(pin[I], sp.dxa, sp.dxb, alpha, buf, I, lane);
+      pack<C, I + 1>();
+    }
+  }
+  template <int C, int I = 0>
+  __device__ __forceinline__ void take() {
+    if constexpr (I < PB && C * PB + I < kNP) {
+      T oa[XPL], ob[XPL];
+      pair_read<MX, V>(buf, I, oa, ob, lane);
+      use<C * PB + I>(oa, ob);
+      take<C, I + 1>();
+    }
+  }
+  template <int C>
+  __device__ __forceinline__ void batch() {
+    if constexpr (C * PB == 18) {  // c_n complete: forward transforms of its three pairs
+      fwd_s();
+    }
+    // FP64 rows have no registers for the next rows during the transforms
+    // (256 a lane): they are loaded while this batch's points are used
+    constexpr bool early = sizeof(V) == 8;
+    constexpr bool more = (C + 1) * PB < kNP;
+    pack<C>();
+    if constexpr (early && more) load<C + 1>();
+    xfft_inv<MX, PB, V>(buf, tw, lane);
+    if constexpr (!early && more) load<C + 1>();
+    take<C>();
+    wave_sync();
+  }
   template <int Q>
-  __device__ __forceinline__ void step() {
-    constexpr PairSpec sp = poly_pair(Q);
-    if constexpr (Q + 1 < kNP) {
-      constexpr PairSpec nx = poly_pair(Q + 1);
-      pair_load<MX, V>(pin[(Q + 1) & 1], rowp(nx.fa), rowp(nx.fb), nxh, lane);
-    }
-    if constexpr (Q == 18) {  // c_n complete: forward transforms of its three pairs
-      fwd_s<0>();
-      fwd_s<2>();
-      fwd_s<4>();
-    }
-    T oa[XPL], ob[XPL];
-    pair_inv<MX, V>(pin[Q & 1], sp.dxa, sp.dxb, nxh, alpha, buf, scr, tw, lane, oa, ob);
+  __device__ __forceinline__ void use(const T (&oa)[XPL], const T (&ob)[XPL]) {
     if (capg) {  // g[3 i + k] = du_i/dx_k
       if constexpr (Q == 3) { cap(capg, 0, oa); cap(capg, 3, ob); }
       if constexpr (Q == 4) { cap(capg, 6, oa); cap(capg, 1, ob); }
@@ -788,46 +767,68 @@ struct PolyRow {
 #pragma unroll
       for (int e = 0; e < 6; ++e) asm volatile("" : "+v"(s[m][e])::"memory");
   }
-  template <int E>
+  // forward transforms of c_n, three pairs
   __device__ __forceinline__ void fwd_s() {
-    T sa[XPL], sb[XPL];
 #pragma unroll
-    for (int m = 0; m < XPL; ++m) { sa[m] = s[m][E]; sb[m] = s[m][E + 1]; }
-    xrow_pair_fwd<MX, V>(sa, sb, orow(E), orow(E + 1), nxh, buf, scr, tw, lane);
+    for (int p0 = 0; p0 < 3; p0 += PB) {
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        if (p0 + i >= 3) continue;
+        T sa[XPL], sb[XPL];
+#pragma unroll
+        for (int m = 0; m < XPL; ++m) { sa[m] = s[m][2 * (p0 + i)]; sb[m] = s[m][2 * (p0 + i) + 1]; }
+        pair_write<MX, V>(buf, i, sa, sb, lane);
+      }
+      xfft_fwd<MX, PB, V>(buf, tw, lane);
+#pragma unroll
+      for (int i = 0; i < PB; ++i)
+        if (p0 + i < 3) xline_unpack<MX, V>(buf, i, orow(2 * (p0 + i)), orow(2 * (p0 + i) + 1), lane);
+      wave_sync();
+    }
   }
   // Peterlin stress str = f C - I and its forward transforms
-  template <int E>
   __device__ __forceinline__ void fwd_str() {
-    T sa[XPL], sb[XPL];
 #pragma unroll
-    for (int m = 0; m < XPL; ++m) {
-      const T tr = c[m][0] + c[m][3] + c[m][5];
-      const T fac = ipeter ? (L2 - (T)3) / (L2 - tr) : (T)1;
-      sa[m] = fac * c[m][E] - ((E == 0) ? (T)1 : (T)0);
-      sb[m] = fac * c[m][E + 1] - ((E + 1 == 3 || E + 1 == 5) ? (T)1 : (T)0);
+    for (int p0 = 0; p0 < 3; p0 += PB) {
+#pragma unroll
+      for (int i = 0; i < PB; ++i) {
+        const int E = 2 * (p0 + i);
+        if (E >= 6) continue;
+        T sa[XPL], sb[XPL];
+#pragma unroll
+        for (int m = 0; m < XPL; ++m) {
+          const T tr = c[m][0] + c[m][3] + c[m][5];
+          const T fac = ipeter ? (L2 - (T)3) / (L2 - tr) : (T)1;
+          sa[m] = fac * c[m][E] - ((E == 0) ? (T)1 : (T)0);
+          sb[m] = fac * c[m][E + 1] - ((E + 1 == 3 || E + 1 == 5) ? (T)1 : (T)0);
+        }
+        if (caps) { cap(caps, E, sa); cap(caps, E + 1, sb); }
+        pair_write<MX, V>(buf, i, sa, sb, lane);
+      }
+      xfft_fwd<MX, PB, V>(buf, tw, lane);
+#pragma unroll
+      for (int i = 0; i < PB; ++i)
+        if (p0 + i < 3) xline_unpack<MX, V>(buf, i, orow(6 + 2 * (p0 + i)), orow(7 + 2 * (p0 + i)), lane);
+      wave_sync();
     }
-    if (caps) { cap(caps, E, sa); cap(caps, E + 1, sb); }
-    xrow_pair_fwd<MX, V>(sa, sb, orow(6 + E), orow(7 + E), nxh, buf, scr, tw, lane);
   }
-  template <int... Q>
-  __device__ __forceinline__ void run(std::integer_sequence<int, Q...>) {
-    (step<Q>(), ...);
+  template <int... C>
+  __device__ __forceinline__ void run(std::integer_sequence<int, C...>) {
+    (batch<C>(), ...);
   }
 };
 
-// Rows up to MX = 288 run two waves per SIMD (256 registers: FP64 spills 3
-// values at MX = 288, FP32 none). At MX = 384, FP64 also runs two (92 bytes a
-// lane spilled: 22 % faster than one wave per SIMD holding 280 registers) and
-// FP32 three (36 bytes a lane spilled; 7 % faster than two).
+// Two waves per SIMD (256 registers: FP64 spills 52 bytes a lane at MX = 288,
+// 208 at 384; one wave per SIMD without spills is slower, the LDS of two
+// blocks a CU allows no third), FP32 rows of 288 and 384 points three.
 template <int MX, typename V>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MX <= 288 ? 2 : (sizeof(V) == 8 ? 3 : 2))))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MX >= 288 && sizeof(V) == 8 ? 3 : 2)))
 void k_xplane_poly(PolyPlaneArgs A) {
   using T = typename Scal<V>::T;
   constexpr int WPB = 4;
   extern __shared__ __align__(16) unsigned char smraw[];
   V* sm = reinterpret_cast<V*>(smraw);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int BL = FFTBuf<MX>::len;
   V* tw = sm;
   for (int e = threadIdx.x; e < MX; e += WPB * 64) tw[e] = static_cast<const V*>(A.twX)[e];
   __syncthreads();
@@ -837,15 +838,13 @@ void k_xplane_poly(PolyPlaneArgs A) {
   R.U = static_cast<const V*>(A.U);
   R.ZP = static_cast<const V*>(A.ZP);
   R.ZF = static_cast<V*>(A.ZFP);
-  R.nxh = A.nxh;
   R.plane = (size_t)A.nyp * A.mz * A.nxh;
   R.roff = ((size_t)y * A.mz + z) * A.nxh;
   R.lane = lane;
   R.ipeter = A.ipeter;
   R.alpha = A.alpha;
   R.L2 = (T)A.L2;
-  R.buf = sm + MX + (size_t)wv * 2 * BL;
-  R.scr = R.buf + BL;
+  R.buf = sm + MX + (size_t)wv * PolyRow<MX, V>::PB * XFft<MX>::BUF;
   R.tw = tw;
   R.capg = A.capg;
   R.caps = A.caps;
@@ -855,14 +854,9 @@ void k_xplane_poly(PolyPlaneArgs A) {
   for (int m = 0; m < PolyRow<MX, V>::XPL; ++m)
 #pragma unroll
     for (int e = 0; e < 6; ++e) R.s[m][e] = (T)0;
-  {
-    constexpr PairSpec p0 = poly_pair(0);
-    pair_load<MX, V>(R.pin[0], R.rowp(p0.fa), R.rowp(p0.fb), R.nxh, lane);
-  }
-  R.run(std::make_integer_sequence<int, kNP>{});
-  R.template fwd_str<0>();
-  R.template fwd_str<2>();
-  R.template fwd_str<4>();
+  R.template load<0>();
+  R.run(std::make_integer_sequence<int, (kNP + PolyRow<MX, V>::PB - 1) / PolyRow<MX, V>::PB>{});
+  R.fwd_str();
 }
 
 // Velocity gradient on one row of the 3/2 grid, for the closure features and
@@ -873,6 +867,7 @@ void k_xplane_poly(PolyPlaneArgs A) {
 // i kx w, wz = i kx v - Du) and continuity:
 //   du/dy = dv/dx - wz,  du/dz = wy + dw/dx,  dv/dy = -du/dx - dw/dz,
 //   dw/dy = wx + dv/dz.
+template <int MX> constexpr int kSwirlLines = xlines<MX, 4>();  // 4 or 2
 template <int MX, typename V>
 __global__ __launch_bounds__(256) void k_xplane_swirl(PolyPlaneArgs A) {
   using T = typename Scal<V>::T;
@@ -881,10 +876,9 @@ __global__ __launch_bounds__(256) void k_xplane_swirl(PolyPlaneArgs A) {
   extern __shared__ __align__(16) unsigned char smraw[];
   V* sm = reinterpret_cast<V*>(smraw);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int BL = FFTBuf<MX>::len;
+  using XF = XFft<MX>;
   V* tw = sm;
-  V* buf = sm + MX + (size_t)wv * 2 * BL;
-  V* scr = buf + BL;
+  V* buf = sm + MX + (size_t)wv * kSwirlLines<MX> * XF::BUF;
   for (int e = threadIdx.x; e < MX; e += WPB * 64) tw[e] = static_cast<const V*>(A.twX)[e];
   __syncthreads();
   const int row = blockIdx.x * WPB + wv;  // grid covers nyp * mz rows exactly
@@ -898,15 +892,29 @@ __global__ __launch_bounds__(256) void k_xplane_swirl(PolyPlaneArgs A) {
   auto zrow = [&](int f) { return ZP + (size_t)f * plane + roff; };
   T g[9][XPL];  // g[3 i + k] = d u_i / d x_k
   T ox[XPL], oy[XPL], oz[XPL];
-  PairIn<MX, V> pin;
-  pair_load<MX, V>(pin, urow(0), urow(1), nxh, lane);
-  pair_inv<MX, V>(pin, true, true, nxh, A.alpha, buf, scr, tw, lane, g[0], g[3]);
-  pair_load<MX, V>(pin, urow(2), urow(3), nxh, lane);
-  pair_inv<MX, V>(pin, true, false, nxh, A.alpha, buf, scr, tw, lane, g[6], ox);
-  pair_load<MX, V>(pin, urow(4), urow(5), nxh, lane);
-  pair_inv<MX, V>(pin, false, false, nxh, A.alpha, buf, scr, tw, lane, oy, oz);
-  pair_load<MX, V>(pin, zrow(A.gz), zrow(A.gz + 1), nxh, lane);
-  pair_inv<MX, V>(pin, false, false, nxh, A.alpha, buf, scr, tw, lane, g[5], g[8]);
+  constexpr int PB = kSwirlLines<MX>;  // pairs per batch
+  PairIn<MX, V> pin[4];
+  pair_load<MX, V>(pin[0], urow(0), urow(1), lane);
+  pair_load<MX, V>(pin[1], urow(2), urow(3), lane);
+  pair_load<MX, V>(pin[2], urow(4), urow(5), lane);
+  pair_load<MX, V>(pin[3], zrow(A.gz), zrow(A.gz + 1), lane);
+  pair_pack<MX, V>(pin[0], true, true, A.alpha, buf, 0, lane);
+  pair_pack<MX, V>(pin[1], true, false, A.alpha, buf, 1, lane);
+  if constexpr (PB == 2) {
+    xfft_inv<MX, PB, V>(buf, tw, lane);
+    pair_read<MX, V>(buf, 0, g[0], g[3], lane);
+    pair_read<MX, V>(buf, 1, g[6], ox, lane);
+    wave_sync();
+  }
+  pair_pack<MX, V>(pin[2], false, false, A.alpha, buf, 2 % PB, lane);
+  pair_pack<MX, V>(pin[3], false, false, A.alpha, buf, 3 % PB, lane);
+  xfft_inv<MX, PB, V>(buf, tw, lane);
+  if constexpr (PB == 4) {
+    pair_read<MX, V>(buf, 0, g[0], g[3], lane);
+    pair_read<MX, V>(buf, 1, g[6], ox, lane);
+  }
+  pair_read<MX, V>(buf, 2 % PB, oy, oz, lane);
+  pair_read<MX, V>(buf, 3 % PB, g[5], g[8], lane);
 #pragma unroll
   for (int m = 0; m < XPL; ++m) {
     g[1][m] = g[3][m] - oz[m];
@@ -962,10 +970,9 @@ __global__ __launch_bounds__(256) void k_mr_xinv(MrLapArgs A) {
   extern __shared__ __align__(16) unsigned char smraw[];
   V* sm = reinterpret_cast<V*>(smraw);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int BL = FFTBuf<MX>::len;
+  using XF = XFft<MX>;
   V* tw = sm;
-  V* buf = sm + MX + (size_t)wv * 2 * BL;
-  V* scr = buf + BL;
+  V* buf = sm + MX + (size_t)wv * 2 * XF::BUF;
   for (int e = threadIdx.x; e < MX; e += WPB * 64) tw[e] = static_cast<const V*>(A.twX)[e];
   __syncthreads();
   const int row = blockIdx.x * WPB + wv;  // grid covers nyp * mz rows exactly
@@ -975,11 +982,14 @@ __global__ __launch_bounds__(256) void k_mr_xinv(MrLapArgs A) {
   const size_t roff = ((size_t)y * A.mz + z) * nxh;
   const V* LZ = static_cast<const V*>(A.LZ);
   T a[XPL], b[XPL], c[XPL], d[XPL];
-  PairIn<MX, V> pin;
-  pair_load<MX, V>(pin, LZ + roff, LZ + plane + roff, nxh, lane);
-  pair_inv<MX, V>(pin, false, false, nxh, A.alpha, buf, scr, tw, lane, a, b);
-  pair_load<MX, V>(pin, LZ + 2 * plane + roff, LZ + 2 * plane + roff, nxh, lane);
-  pair_inv<MX, V>(pin, false, false, nxh, A.alpha, buf, scr, tw, lane, c, d);
+  PairIn<MX, V> pin[2];
+  pair_load<MX, V>(pin[0], LZ + roff, LZ + plane + roff, lane);
+  pair_load<MX, V>(pin[1], LZ + 2 * plane + roff, LZ + 2 * plane + roff, lane);
+  pair_pack<MX, V>(pin[0], false, false, A.alpha, buf, 0, lane);
+  pair_pack<MX, V>(pin[1], false, false, A.alpha, buf, 1, lane);
+  xfft_inv<MX, 2, V>(buf, tw, lane);
+  pair_read<MX, V>(buf, 0, a, b, lane);
+  pair_read<MX, V>(buf, 1, c, d, lane);
   const size_t P = (size_t)A.nyp * A.mz * MX;
   const size_t prow = ((size_t)y * A.mz + z) * MX;
 #pragma unroll
@@ -1003,10 +1013,9 @@ __global__ __launch_bounds__(256) void k_xrow_fwd_str(PolyPlaneArgs A) {
   extern __shared__ __align__(16) unsigned char smraw[];
   V* sm = reinterpret_cast<V*>(smraw);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  constexpr int BL = FFTBuf<MX>::len;
+  using XF = XFft<MX>;
   V* tw = sm;
-  V* buf = sm + MX + (size_t)wv * 2 * BL;
-  V* scr = buf + BL;
+  V* buf = sm + MX + (size_t)wv * xlines<MX, 3>() * XF::BUF;
   for (int e = threadIdx.x; e < MX; e += WPB * 64) tw[e] = static_cast<const V*>(A.twX)[e];
   __syncthreads();
   const int row = blockIdx.x * WPB + wv;
@@ -1014,23 +1023,36 @@ __global__ __launch_bounds__(256) void k_xrow_fwd_str(PolyPlaneArgs A) {
   const size_t P = (size_t)A.nyp * A.mz * MX, prow = ((size_t)y * A.mz + z) * MX;
   const size_t plane = (size_t)A.nyp * A.mz * A.nxh, roff = ((size_t)y * A.mz + z) * A.nxh;
   V* ZF = static_cast<V*>(A.ZFP);
+  constexpr int PB = xlines<MX, 3>();
 #pragma unroll
-  for (int e = 0; e < 6; e += 2) {
-    T sa[XPL], sb[XPL];
+  for (int p0 = 0; p0 < 3; p0 += PB) {
 #pragma unroll
-    for (int m = 0; m < XPL; ++m) {
-      const int x = lane + 64 * m;
-      sa[m] = (x < MX) ? (T)A.caps[(size_t)e * P + prow + x] : (T)0;
-      sb[m] = (x < MX) ? (T)A.caps[(size_t)(e + 1) * P + prow + x] : (T)0;
+    for (int i = 0; i < PB; ++i) {
+      const int e = 2 * (p0 + i);
+      if (e >= 6) continue;
+      T sa[XPL], sb[XPL];
+#pragma unroll
+      for (int m = 0; m < XPL; ++m) {
+        const int x = lane + 64 * m;
+        sa[m] = (x < MX) ? (T)A.caps[(size_t)e * P + prow + x] : (T)0;
+        sb[m] = (x < MX) ? (T)A.caps[(size_t)(e + 1) * P + prow + x] : (T)0;
+      }
+      pair_write<MX, V>(buf, i, sa, sb, lane);
     }
-    xrow_pair_fwd<MX, V>(sa, sb, ZF + (size_t)(6 + e) * plane + roff, ZF + (size_t)(7 + e) * plane + roff, A.nxh,
-                         buf, scr, tw, lane);
+    xfft_fwd<MX, PB, V>(buf, tw, lane);
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int e = 2 * (p0 + i);
+      if (e < 6)
+        xline_unpack<MX, V>(buf, i, ZF + (size_t)(6 + e) * plane + roff, ZF + (size_t)(7 + e) * plane + roff, lane);
+    }
+    wave_sync();
   }
 }
 
 template <int MX, int MZ, typename V>
 static hipError_t closure_fwd_impl(const PolyPlaneArgs& pa, hipStream_t s) {
-  const size_t xlds = (size_t)(MX + 4 * 2 * FFTBuf<MX>::len) * sizeof(V);
+  const size_t xlds = xfft_lds<MX, V>(4, xlines<MX, 3>());
   hipLaunchKernelGGL((k_xrow_fwd_str<MX, V>), dim3(pa.nyp * pa.mz / 4), dim3(256), xlds, s, pa);
   PlaneArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -1057,7 +1079,7 @@ static hipError_t swirl_plane_impl(const PolyPlaneArgs& pa, bool zstage, hipStre
     a.Z = pa.ZP;
     launch_zinv<MZ, 2, V>(a, s);
   }
-  const size_t xlds = (size_t)(MX + 4 * 2 * FFTBuf<MX>::len) * sizeof(V);
+  const size_t xlds = xfft_lds<MX, V>(4, kSwirlLines<MX>);
   hipLaunchKernelGGL((k_xplane_swirl<MX, V>), dim3(pa.nyp * pa.mz / 4), dim3(256), xlds, s, pa);
   return hipGetLastError();
 }
@@ -1072,7 +1094,7 @@ static hipError_t mr_lap_plane_impl(const MrLapArgs& la, hipStream_t s) {
   a.dzmask = 0u;
   a.Z = la.LZ;
   launch_zinv<MZ, 3, V>(a, s);
-  const size_t xlds = (size_t)(MX + 4 * 2 * FFTBuf<MX>::len) * sizeof(V);
+  const size_t xlds = xfft_lds<MX, V>(4, 2);
   hipLaunchKernelGGL((k_mr_xinv<MX, V>), dim3(la.nyp * la.mz / 4), dim3(256), xlds, s, la);
   return hipGetLastError();
 }
@@ -1097,7 +1119,7 @@ static hipError_t poly_plane_impl(const PolyPlaneArgs& pa, hipStream_t s) {
     a.Z = static_cast<V*>(pa.ZP) + (size_t)8 * g * zb;
     launch_zinv<MZ, 8, V>(a, s);
   }
-  const size_t xlds = (size_t)(MX + 4 * 2 * FFTBuf<MX>::len) * sizeof(V);
+  const size_t xlds = xfft_lds<MX, V>(4, (PolyRow<MX, V>::PB));
   hipLaunchKernelGGL((k_xplane_poly<MX, V>), dim3(pa.nyp * pa.mz / 4), dim3(256), xlds, s, pa);
   // forward z of the 12 outputs, 4 per launch
   for (int g = 0; g < 3; ++g) {
@@ -1117,7 +1139,7 @@ static hipError_t plane_impl(const PlaneArgs& a, hipStream_t s, bool inverse_par
       hipLaunchKernelGGL((k_ibdrag<MX, V>), dim3((a.nsrc + 3) / 4), dim3(256), 0, s, a);
     if (ev) hipEventRecord(ev[1], s);
     constexpr int WPB = 4;
-    const size_t xlds = (size_t)(MX + WPB * 2 * FFTBuf<MX>::len) * sizeof(V);
+    const size_t xlds = xfft_lds<MX, V>(WPB, xplane_lines<MX, NFIN, NFOUT>());
     if (a.tune == 1)
       hipLaunchKernelGGL((k_xplane<MX, NFIN, NFOUT, WPB, V, 1>), dim3(a.nyp * (a.mz / (2 * WPB))), dim3(WPB * 64),
                          xlds, s, a);
@@ -1174,7 +1196,7 @@ static hipError_t plane_batch_impl(const PlaneArgs& a, const PlaneArgs* dA, int 
     hipLaunchKernelGGL((k_zinv_batch<MZ, NFIN, V>), dim3(grid, nmem), dim3(512), zlds, s, dA);
   }
   constexpr int WPB = 4;
-  const size_t xlds = (size_t)(MX + WPB * 2 * FFTBuf<MX>::len) * sizeof(V);
+  const size_t xlds = xfft_lds<MX, V>(WPB, xplane_lines<MX, NFIN, NFOUT>());
   const dim3 gx(a.nyp * (a.mz / (2 * WPB)), nmem);
   if (a.tune == 1)
     hipLaunchKernelGGL((k_xplane_batch<MX, NFIN, NFOUT, WPB, V, 1>), gx, dim3(WPB * 64), xlds, s, dA);
