@@ -770,22 +770,6 @@ __device__ __forceinline__ PFN<NY> phirhs(const PFN<NY>& v, const PFN<NY>& d2v, 
 }
 
 
-// mean over y of a Chebyshev series: sum over even n of a_n / (1 - n^2)
-template <int NY>
-__device__ __forceinline__ double pf_bulk(const PFN<NY>& f, int lane) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-  double v = 0.0;
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g = s * WAVE + lane;
-    const double n = 2.0 * g;
-    const double vs = (g < L) ? f.a[s].x / (1.0 - n * n) : 0.0;
-    v = s ? v + vs : vs;
-  }
-  v = wave_sum(v);
-  return v + f.e.x / (1.0 - (double)NY * (double)NY);
-}
-
 // ------------------------------------------------ shared by the pencil kernels --
 constexpr int PW = 8;  // wavefronts (pencils) per workgroup
 
@@ -794,92 +778,11 @@ __device__ __forceinline__ V* wave_lds(V* smem, int wv) {
   // twiddles [2NY], then two padded FFT buffers of length 2NY per wave
   return smem + 2 * NY + (size_t)wv * 2 * FFTBuf<2 * NY>::len;
 }
-// ------------------------------------------------ block-staged tiles --
-// The PWS consecutive pencils p0 .. p0+PWS-1 of a block, rows y = 0..NY of
-// a field laid out [y][pencil], staged through an LDS tile [NY+1][PWS+1]
-// (one pad element per row): the block's global accesses then cover whole
-// rows of PWS pencils (64 bytes per row for FP64), and each wave takes its
-// own pencil's column from the tile.  Thread t moves elements
-// e = t + k PWS*64 (row e / PWS, pencil e % PWS).  Four pencils per block
-// keep the staged step kernel within half the CU's LDS, so that two blocks
-// share a CU and one computes while the other waits at a block barrier.
-constexpr int PWS = 4;
-constexpr int TLD = PWS + 1;
-template <int NY>
-struct TileG {
-  static constexpr int ROWS = NY + 1, NEL = ROWS * PWS, LEN = ROWS * TLD;
-  static constexpr int PER = (NEL + PWS * WAVE - 1) / (PWS * WAVE);
-};
-template <int NY, typename E>
-__device__ __forceinline__ void tile_fetch(const E* __restrict__ F, size_t P, int p0, E (&r)[TileG<NY>::PER]) {
-  using G = TileG<NY>;
-#pragma unroll
-  for (int k = 0; k < G::PER; ++k) {
-    const int e = (int)threadIdx.x + k * PWS * WAVE;
-    const int y = e / PWS, w = e % PWS;
-    r[k] = (e < G::NEL && (size_t)(p0 + w) < P) ? F[(size_t)y * P + p0 + w] : vzero<E>();
-  }
-}
-template <int NY, typename E>
-__device__ __forceinline__ void tile_put(E* t, const E (&r)[TileG<NY>::PER]) {
-  using G = TileG<NY>;
-#pragma unroll
-  for (int k = 0; k < G::PER; ++k) {
-    const int e = (int)threadIdx.x + k * PWS * WAVE;
-    if (e < G::NEL) t[(e / PWS) * TLD + e % PWS] = r[k];
-  }
-}
-template <int NY, typename E>
-__device__ __forceinline__ void tile_store(const E* t, E* __restrict__ F, size_t P, int p0) {
-  using G = TileG<NY>;
-#pragma unroll
-  for (int k = 0; k < G::PER; ++k) {
-    const int e = (int)threadIdx.x + k * PWS * WAVE;
-    const int y = e / PWS, w = e % PWS;
-    if (e < G::NEL && (size_t)(p0 + w) < P) F[(size_t)y * P + p0 + w] = t[y * TLD + w];
-  }
-}
-// physical values of column wv of a tile in the transfer precision
-template <int NY, typename V>
-__device__ __forceinline__ PhysN<NY, V> tile_phys(const V* t, int wv, int lane) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-  PhysN<NY, V> q;
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g0 = s * WAVE + lane;
-    const int g = g0 < L ? g0 : L - 1;
-    q.a[s] = t[(2 * g) * TLD + wv];
-    q.b[s] = t[(2 * g + 1) * TLD + wv];
-  }
-  q.e = t[NY * TLD + wv];
-  return q;
-}
-// inverse transform of f into column wv of a transfer tile (zeros: zero column)
-template <int NY, typename V>
-__device__ __forceinline__ void cheb_to_phys_tile(const PFN<NY>& f, V* buf, V* scr, const V* tw, int lane, V* t,
-                                                  int wv) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-  const V* r = cheb_to_phys<NY, V>(f, buf, scr, tw, lane);
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g = s * WAVE + lane;
-    if (g < L) {
-      t[(2 * g) * TLD + wv] = r[fpad(2 * g)];
-      t[(2 * g + 1) * TLD + wv] = r[fpad(2 * g + 1)];
-    }
-  }
-  if (lane == 0) t[NY * TLD + wv] = r[fpad(NY)];
-  wave_sync();
-}
-template <int NY, typename V>
-__device__ __forceinline__ void tile_col_zero(V* t, int wv, int lane) {
-  for (int y = lane; y <= NY; y += WAVE) t[y * TLD + wv] = vzero<V>();
-}
-
 // Pencil group of block b of nb: blocks are dispatched round-robin over the
-// 8 XCDs (block b on XCD b % 8), each with its own L2; groups 4k .. 4k+3
-// share the cache lines of every [y][pencil] row (64 bytes per group for
-// FP64, 32 for FP32), so they go to blocks b, b+8, b+16, b+24 of one XCD.
+// 8 XCDs (block b on XCD b % 8), each with its own L2; neighbouring groups
+// share the pages and, where a row's line is wider than a group, the cache
+// lines of every [y][pencil] row, so groups 4k .. 4k+3 go to blocks b, b+8,
+// b+16, b+24 of one XCD.
 // A bijection of 0..nb-1 (blocks past the last multiple of 32 keep their
 // index).
 __device__ __forceinline__ int xcd_group(int b, int nb) {
@@ -887,27 +790,6 @@ __device__ __forceinline__ int xcd_group(int b, int nb) {
   const int x = b % 8, s = b / 8;
   return (s / 4) * 32 + x * 4 + s % 4;
 }
-
-// LDS plan of the staged step kernel (bytes): twiddles, then a region used
-// as [FFT buffers | two nonlinear-term tiles] while the nonlinear terms are
-// transformed (two rounds of two) and as [FFT buffers | transfer tiles] for
-// the inverse transforms; at most 54 KB, so that three blocks of four waves
-// share a CU (three waves per SIMD at the step kernel's 168 registers).
-template <int NY, typename V, bool SCALAR>
-struct StepLds {
-  // three blocks per CU up to ny = 128, two at ny = 192
-  static constexpr size_t CAP = (NY <= 128 ? 54 : 80) * 1024;
-  static constexpr size_t TWB = (size_t)2 * NY * sizeof(V);
-  static constexpr size_t FFT = (size_t)PWS * FFTBuf<2 * NY>::len * sizeof(V);  // one in-place buffer per wave
-  static constexpr size_t TV = (size_t)TileG<NY>::LEN * sizeof(V);
-  static constexpr int NOUT = SCALAR ? 9 : 6;
-  static constexpr int fit = (CAP > TWB + FFT) ? (int)((CAP - TWB - FFT) / TV) : 0;
-  static constexpr int NTS = fit < NOUT ? fit : NOUT;  // transfer tiles per flush
-  static constexpr size_t A1 = FFT + 2 * TV, A3 = FFT + (size_t)NTS * TV;
-  static constexpr size_t REGION = A1 > A3 ? A1 : A3;
-  static constexpr bool ok = NTS >= 3 && TWB + REGION <= CAP && fft_in_place<2 * NY, kChebPlan>();
-  static constexpr size_t bytes = TWB + REGION;
-};
 
 // block-wide copy of the length-2NY twiddles into LDS (before any early exit)
 template <int NY, typename V>
@@ -960,20 +842,5 @@ __device__ __forceinline__ PFN<NY> smooth_apply(const PFN<NY>& f, const double* 
 static inline int nblk(int P) { return (P + PW - 1) / PW; }
 template <int NY, typename V>
 static inline size_t lds_bytes(int waves = PW) { return (size_t)(waves * 2 * FFTBuf<2 * NY>::len + 2 * NY) * sizeof(V); }
-// the step kernel's launch: the staged plan (PWS pencils per block) where
-// it fits, else PW pencils per block with their FFT buffers
-template <int NY, typename V, bool SCALAR, int MODE>
-constexpr bool step_tiled() { return MODE == 0 && StepLds<NY, V, SCALAR>::ok; }
-template <int NY, typename V, bool SCALAR, int MODE>
-static inline size_t step_lds_bytes() {
-  if constexpr (step_tiled<NY, V, SCALAR, MODE>()) return StepLds<NY, V, SCALAR>::bytes;
-  else return lds_bytes<NY, V>();
-}
-template <int NY, typename V, bool SCALAR, int MODE>
-static inline int step_blocks(int P) {
-  return step_tiled<NY, V, SCALAR, MODE>() ? (P + PWS - 1) / PWS : nblk(P);
-}
-template <int NY, typename V, bool SCALAR, int MODE>
-static inline int step_threads() { return (step_tiled<NY, V, SCALAR, MODE>() ? PWS : PW) * 64; }
 
 }  // namespace kmm

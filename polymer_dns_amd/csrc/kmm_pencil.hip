@@ -13,6 +13,7 @@
 // with every pencil operation); the pencil-local ones are applied here.
 #include "kmm_kernels.h"
 #include "kmm_pencil.h"
+#include "kmm_row.h"
 
 namespace kmm {
 
@@ -110,562 +111,273 @@ __global__ __launch_bounds__(PW * 64) void k_green(PencilArgs A, double pb1, dou
 }
 
 // ----------------------------------------------------------- the step --
+// A real Green's function (pairs of values, NY/2 + 1 entries).
+// G: the wavefront's first pencil's, o: the row's offset
 template <int NY>
-__device__ __forceinline__ PFN<NY> green_load(const double2* __restrict__ G, int p, int lane) {
-  constexpr int L = NY / 2;
-  const double2* g = G + (size_t)p * (L + 1);
-  PFN<NY> f = pf_zero<NY>();
+__device__ __forceinline__ void green_add(RP<NY>& v, double2 c, const double2* __restrict__ G, unsigned o, int l) {
+  constexpr int L = RLay<NY>::L, K = RLay<NY>::K;
 #pragma unroll
-  for (int q = 0; q < PLay<NY>::S; ++q) {
-    const int gi = q * WAVE + lane;
-    if (gi < L) { double2 v = g[gi]; f.a[q].x = v.x; f.b[q].x = v.y; }
+  for (int i = 0; i < K; ++i) {
+    const int g = K * l + i;
+    if (RLay<NY>::FULL || g < L) {
+      const double2 q = G[o + g];
+      v.a[i] = cfma(q.x, c, v.a[i]);
+      v.b[i] = cfma(q.y, c, v.b[i]);
+    }
   }
-  f.e.x = g[L].x;
-  return f;
+  v.e = cfma(G[o + L].x, c, v.e);
 }
-
 
 // MODE 0: full step (NL from buffers or FN/GN/SCN), MODE 1: startup
 // (derived fields of the current state only), MODE 2: finish (NL -> FN, GN,
-// SCN, h1n, h3n).
-// TV: occupancy variant picked by the autotuner (0: the compiler's register
-// budget, 2 waves/SIMD at NY = 128; 1: at least 3 waves/SIMD, <= 168 VGPRs)
-// The body of one block of pencils (blk: the block's index along its
-// channel's pencils).
+// SCN, h1n, h3n).  blk: the block's index along its channel's pencils (16 a
+// block, four a wavefront, one per row of 16 lanes: kmm_row.h).
+//
+// Order: the scalar through to its transfer fields, then omega_y, then v, so
+// that at most three pencils and a solve's temporaries are held at a time (two
+// wavefronts per SIMD).  All walls are no-slip or moving walls
+// (Dirichlet rows, checked by the launch), so the mean-flow solves (uzero,
+// solvers.f90:1065-1176) are omega_y's of the (0,0) pencil: u0 and w0 as the
+// real and imaginary part of its unknown.  The z-Nyquist pencil computes on
+// zeros (norm zeroes it, helpers.f90:149-156).
+// The transforms stand in loops that are not unrolled: one copy of their code
+// for the nonlinear terms, one for the scalar's and one for the flow's fields.
 template <int NY, bool SCALAR, int MODE, typename V>
 __device__ __forceinline__ void pencil_body(const PencilArgs& A, int blk) {
-  using PF = PFN<NY>;
+  using RL = RLay<NY>;
+  using PF = RP<NY>;
   extern __shared__ __align__(16) unsigned char smraw[];
   V* smem = reinterpret_cast<V*>(smraw);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int p = blk * PW + wv;
-  const V* twl = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
-  if (p >= A.P) return;
-  V* buf = wave_lds<NY, V>(smem, wv);
-  V* scr = buf + FFTBuf<2 * NY>::len;
+  const V* tw = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
+  const int lane = threadIdx.x & 63, l = lane & 15, row = lane >> 4;
+  const unsigned wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double2* wd = reinterpret_cast<double2*>(smraw + 2 * NY * sizeof(V)) + (size_t)wv * RPW * RL::BUF;
+  V* w = reinterpret_cast<V*>(wd);          // the wavefront's lines in the transfer precision
+  const unsigned P = (unsigned)A.P, p0 = (unsigned)(blk * RWV + wv) * RPW;
+  constexpr unsigned TW = tab_width(NY);
+  const unsigned rt = row * TW;             // the row's table entries from the wavefront's first
   V* const* TT = reinterpret_cast<V* const*>(A.T);
-  const size_t P = (size_t)A.P;
+  V* const* TPD = reinterpret_cast<V* const*>(A.TPD);
   double kx, kz;
   int kxi, kzi;
-  pencil_k(A, p, kx, kz, kxi, kzi);
+  pencil_k(A, (int)p0 + row, kx, kz, kxi, kzi);
   const double k2 = kx * kx + kz * kz;
-  const bool is00 = (kxi == 0 && kzi == 0);
-  const bool nyq = (kzi == A.nzh);
-  const double dy = A.dyde;
-  const int nT = SCALAR ? 9 : 6;
+  const bool is00 = (kxi == 0 && kzi == 0), nyq = (kzi == A.nzh);
+  const double dy = A.dyde, th = A.theta;
+  const bool fromNL = MODE == 2 || (MODE == 0 && A.first_nl);
+  const double sz = A.smooth ? A.smz[kzi] : 1.0;
+  using RV = RowRaw<NY, V>;
+  using RD = RowRaw<NY, double2>;
+  // a nonlinear term's coefficients
+  auto term = [&](const void* F, const double2* TF) -> PF {
+    RV q;
+    rows_fetch<NY, V>(q, static_cast<const V*>(F), P, p0, lane);
+    PF h = rows_to_cheb<NY, V>(q, w, tw, lane);
+    if (TF) h = pf_add(h, pm_load<NY>(TF, p0, wd, lane));  // subforce (helpers.f90:564-606), before smoothing
+    if (A.smooth) r_smooth<NY>(h, A.smy, sz, l);
+    rp_mask_imag(h, is00);
+    rp_mask(h, nyq);
+    return h;
+  };
 
-  if (nyq) {  // norm zeroes the z-Nyquist row (helpers.f90:149-156)
-    PF z = pf_zero<NY>();
-    if (MODE == 0) {
-      pf_store_pm<NY>(A.V, p, lane, z); pf_store_pm<NY>(A.OMY, p, lane, z);
-      pf_store_pm<NY>(A.FNM1, p, lane, z); pf_store_pm<NY>(A.GNM1, p, lane, z);
-      if (SCALAR) { pf_store_pm<NY>(A.TH, p, lane, z); pf_store_pm<NY>(A.SCNM1, p, lane, z); }
+  // ---------------- scalar (main_dns.f90:324-358) ----------------------
+  if (SCALAR) {
+    PF sn, sc;
+    if (MODE != 1) {
+      if (fromNL) {
+        sn = term(A.NLS, nullptr);
+      } else {
+        sn = pm_load<NY>(A.SCN, p0, wd, lane);
+        rp_mask(sn, nyq);
+      }
     }
     if (MODE == 2) {
-      pf_store_pm<NY>(A.FN, p, lane, z); pf_store_pm<NY>(A.GN, p, lane, z);
-      if (SCALAR) pf_store_pm<NY>(A.SCN, p, lane, z);
-    }
-    if (MODE != 2)
-      for (int t = 0; t < nT + 3; ++t) {
-        V* d = (t < nT) ? TT[t] : static_cast<V*>(A.TPD[t - nT]);
-        if (!d) continue;
-        pf_store_zero<NY, V>(d, P, p, lane);
+      pm_store<NY>(A.SCN, p0, wd, lane, sn);
+    } else {
+      sc = pm_load<NY>(A.TH, p0, wd, lane);
+      rp_mask(sc, nyq);
+      if (MODE == 0) {
+        RD qm;
+        pm_fetch<NY>(qm, A.SCNM1, p0, lane);
+        PF rhs = r_cderiv<NY>(r_cderiv<NY>(sc, dy, l), dy, l);
+        PF old = pm_take<NY>(qm, wd, lane);
+        rp_mask(old, nyq);
+        rhs = r_phirhs(sc, rhs, sn, old, k2, A.re, A.diff, A.dt, th);
+        pm_store<NY>(A.SCNM1, p0, wd, lane, sn);
+        sc = r_solve<NY, true>(rhs, k2 + A.gS, dy, A.tabS + (size_t)p0 * TW, rt, czero(), czero(), l);
+        rp_mask_imag(sc, is00);
+        pm_store<NY>(A.TH, p0, wd, lane, sc);
       }
-    return;
+#pragma unroll 1
+      for (int j = 0; j < 3; ++j) {
+        PF o = pf_imul(sc, j == 0 ? kx : kz);
+        if (j == 1) o = r_cderiv<NY>(sc, dy, l);
+        cheb_to_rows<NY, V>(o, w, tw, lane, TT[6 + j], P, p0);
+      }
+    }
   }
 
-  // ---------------- part B: nonlinear terms -> fn, gn, scn (spectral) --
-  PF fn, gn, sn;
-  PF h1m, h3m;  // mean-mode profiles (only used by the (0,0) pencil)
-  if (MODE == 0 || MODE == 2) {
-    if (MODE == 2 || A.first_nl) {
-      const double sz = A.smooth ? A.smz[kzi] : 1.0;
-      // each pencil's load is issued one transform ahead
-      PhysN<NY, V> q1 = phys_load<NY, V>(static_cast<const V*>(A.NL1), P, p, lane);
-      PhysN<NY, V> q3 = phys_load<NY, V>(static_cast<const V*>(A.NL3), P, p, lane);
-      PF h1 = phys_to_cheb<NY, V>(q1, buf, scr, twl, lane);
-      PhysN<NY, V> q2 = phys_load<NY, V>(static_cast<const V*>(A.NL2), P, p, lane);
-      PF h3 = phys_to_cheb<NY, V>(q3, buf, scr, twl, lane);
-      PhysN<NY, V> qs;
-      if (SCALAR) qs = phys_load<NY, V>(static_cast<const V*>(A.NLS), P, p, lane);
-      PF h2 = phys_to_cheb<NY, V>(q2, buf, scr, twl, lane);
-      if (A.TF[0]) {  // polymer force, subforce (helpers.f90:564-606), before smoothing
-        h1 = pf_add(h1, pf_load<NY>(A.TF[0], P, p, lane));
-        h2 = pf_add(h2, pf_load<NY>(A.TF[1], P, p, lane));
-        h3 = pf_add(h3, pf_load<NY>(A.TF[2], P, p, lane));
-      }
-      if (A.smooth) {
-        h1 = smooth_apply<NY>(h1, A.smy, sz, lane);
-        h2 = smooth_apply<NY>(h2, A.smy, sz, lane);
-        h3 = smooth_apply<NY>(h3, A.smy, sz, lane);
-      }
-      if (is00) { h1 = pf_real(h1); h2 = pf_real(h2); h3 = pf_real(h3); }
-      h1m = h1;
-      h3m = h3;
-      // nonlin (solvers.f90:1497-1572)
-      PF x = pf_add(pf_imul(h3, kz), pf_imul(h1, kx));
-      PF dx = cderiv<NY>(x, dy, lane);
-      fn = pf_sub(pf_scale(h2, -k2), dx);
-      gn = pf_sub(pf_imul(h1, kz), pf_imul(h3, kx));
-      if (SCALAR) {
-        sn = phys_to_cheb<NY, V>(qs, buf, scr, twl, lane);
-        if (A.smooth) sn = smooth_apply<NY>(sn, A.smy, sz, lane);
-        if (is00) sn = pf_real(sn);
-      }
-      if (is00) {
-        // main_dns.f90:748-751 (h1n = Re gn(:,1,1), h3n = Re omz(:,1,1))
-        if (MODE == 2) {
-          pf_store_real<NY>(A.h1n, lane, h1m);
-          pf_store_real<NY>(A.h3n, lane, h3m);
+  // ---------------- nonlinear terms -> fn, gn (spectral) ---------------
+  // nonlin (solvers.f90:1497-1572); gn of the (0,0) pencil: the mean terms
+  // h1 + i h3 (main_dns.f90:748-751)
+  PF fn, gn;
+  if (MODE != 1) {
+    if (fromNL) {
+#pragma unroll 1
+      for (int j = 0; j < 3; ++j) {
+        const PF h = term(j == 0 ? A.NL1 : j == 1 ? A.NL3 : A.NL2, j == 0 ? A.TF[0] : j == 1 ? A.TF[2] : A.TF[1]);
+        if (j == 0) {
+          fn = pf_imul(h, kx);
+          gn = pf_imul(h, kz);
+          if (is00) gn = h;
+        } else if (j == 1) {
+          fn = pf_add(fn, pf_imul(h, kz));
+          gn = pf_sub(gn, pf_imul(h, is00 ? -1.0 : kx));
+        } else {
+          fn = pf_sub(pf_scale(h, -k2), r_cderiv<NY>(fn, dy, l));
         }
       }
       if (MODE == 2) {
-        pf_store_pm<NY>(A.FN, p, lane, fn);
-        pf_store_pm<NY>(A.GN, p, lane, gn);
-        if (SCALAR) pf_store_pm<NY>(A.SCN, p, lane, sn);
+        pm_store<NY>(A.FN, p0, wd, lane, fn);
+        if (is00) mean_store<NY>(A.h1n, A.h3n, gn, l);
+        rp_mask(gn, is00);
+        pm_store<NY>(A.GN, p0, wd, lane, gn);
         return;
       }
     } else {
-      fn = pf_load_pm<NY>(A.FN, p, lane);
-      gn = pf_load_pm<NY>(A.GN, p, lane);
-      if (SCALAR) sn = pf_load_pm<NY>(A.SCN, p, lane);
-      if (is00) { h1m = pf_load_real<NY>(A.h1n, lane); h3m = pf_load_real<NY>(A.h3n, lane); }
+      fn = pm_load<NY>(A.FN, p0, wd, lane);
+      gn = pm_load<NY>(A.GN, p0, wd, lane);
+      if (is00) gn = mean_load<NY>(A.h1n, A.h3n, l);
+      rp_mask(fn, nyq);
+      rp_mask(gn, nyq);
     }
   }
 
-  const double th = A.theta;
-  // ---------------- scalar (main_dns.f90:324-358) ----------------------
-  PF sc;
-  if (SCALAR) {
-    sc = pf_load_pm<NY>(A.TH, p, lane);
-    if (MODE == 0) {
-      PF scnm1 = pf_load_pm<NY>(A.SCNM1, p, lane);
-      PF d1 = cderiv<NY>(sc, dy, lane);
-      PF d2 = cderiv<NY>(d1, dy, lane);
-      PF rhs = phirhs<NY>(sc, d2, sn, scnm1, k2, A.re, A.diff, A.dt, th);
-      pf_store_pm<NY>(A.SCNM1, p, lane, sn);
-      auto tt = [dy](int n) -> double { return dy * (double)n * (double)n; };
-      auto tb = [dy](int n) -> double { double v = dy * (double)n * (double)n; return (n & 1) ? -v : v; };
-      sc = tau_penta<NY>(rhs, k2 + A.gS, dy, A.tabS + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-      if (is00) sc = pf_real(sc);
-      pf_store_pm<NY>(A.TH, p, lane, sc);
-    }
-  }
-
-  // ---------------- v and omega_y (main_dns.f90:360-502) ---------------
-  PF v, omy;
-  PF u0p, w0p;
+  // ---------------- omega_y and the mean flow, v (main_dns.f90:360-502) --
+  PF omy = pm_load<NY>(A.OMY, p0, wd, lane), v;
+  rp_mask(omy, nyq || is00);
   if (MODE == 0) {
-    if (!is00) {
-      v = pf_load_pm<NY>(A.V, p, lane);
-      PF fnm1 = pf_load_pm<NY>(A.FNM1, p, lane);
-      PF d1 = cderiv<NY>(v, dy, lane);
-      PF d2 = cderiv<NY>(d1, dy, lane);
-      PF phi = pf_sub(d2, pf_scale(v, k2));
-      d1 = cderiv<NY>(phi, dy, lane);
-      d2 = cderiv<NY>(d1, dy, lane);
-      PF rhs = phirhs<NY>(phi, d2, fn, fnm1, k2, A.re, 1.0, A.dt, th);
-      pf_store_pm<NY>(A.FNM1, p, lane, fn);
-      phi = tau_solve<NY>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p * tab_width(NY), czero(), czero(), 0, lane);
-      PF vp = tau_solve<NY>(phi, k2, dy, A.tabP + (size_t)p * tab_width(NY), czero(), czero(), 0, lane);
-      double2 vt, vb;
-      wall_derivs<NY>(vp, dy, lane, vt, vb);
-      const double4 g = A.gk[p];
-      double2 c1 = cadd(cscale(vb, g.x), cscale(vt, g.y));
-      double2 c2 = cadd(cscale(vb, g.z), cscale(vt, g.w));
-      v = pf_add(vp, pf_add(pf_cmul_real(c1, green_load<NY>(A.G1, p, lane)),
-                            pf_cmul_real(c2, green_load<NY>(A.G2, p, lane))));
-      omy = pf_load_pm<NY>(A.OMY, p, lane);
-      PF gnm1 = pf_load_pm<NY>(A.GNM1, p, lane);
-      PF e1 = cderiv<NY>(omy, dy, lane);
-      PF e2 = cderiv<NY>(e1, dy, lane);
-      PF orhs = phirhs<NY>(omy, e2, gn, gnm1, k2, A.re, 1.0, A.dt, th);
-      pf_store_pm<NY>(A.GNM1, p, lane, gn);
-      const double atu = A.atu, btu = A.btu, abu = A.abu, bbu = A.bbu;
-      auto tt = [=](int n) -> double { return atu + dy * btu * (double)n * (double)n; };
-      auto tb = [=](int n) -> double { double t = abu + dy * bbu * (double)n * (double)n; return (n & 1) ? -t : t; };
-      omy = tau_penta<NY>(orhs, k2 + A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-      pf_store_pm<NY>(A.V, p, lane, v);
-      pf_store_pm<NY>(A.OMY, p, lane, omy);
-    } else {
-      // (0,0): v = 0 (veloc), omega_y = 0, fnm1 = fn = 0, gnm1 = gn = 0,
-      // and the mean-flow solves (uzero, solvers.f90:1065-1176).
-      v = pf_zero<NY>();
-      omy = pf_zero<NY>();
-      pf_store_pm<NY>(A.V, p, lane, v);
-      pf_store_pm<NY>(A.OMY, p, lane, omy);
-      pf_store_pm<NY>(A.FNM1, p, lane, pf_zero<NY>());
-      pf_store_pm<NY>(A.GNM1, p, lane, pf_zero<NY>());
-      for (int w = 0; w < 2; ++w) {
-        double* um = w ? A.w0 : A.u0;
-        double* hl = w ? A.h3nm1 : A.h1nm1;
-        double* hn = w ? A.h3n : A.h1n;
-        const PF& hcur = w ? h3m : h1m;
-        PF u = pf_load_real<NY>(um, lane);
-        PF hlp = pf_load_real<NY>(hl, lane);
-        PF d1 = cderiv<NY>(u, dy, lane);
-        PF d2 = cderiv<NY>(d1, dy, lane);
-        // wrk1 = -re u0/(dt th) - re (3 h1 - h1l)/(2 th) - (1-th)/th u0''
-        PF r = pf_scale(u, -A.re / (A.dt * th));
-        r = pf_axpy(-3.0 * A.re / (2.0 * th), hcur, r);
-        r = pf_axpy(A.re / (2.0 * th), hlp, r);
-        r = pf_axpy(-(1.0 - th) / th, d2, r);
-        // psolve1d with mixedbc1d rows (correct bottom sign); w0 uses btu
-        // (quirk of solvers.f90:1173).
-        const double at = w ? A.atw : A.atu, bt = A.btu, ab = w ? A.abw : A.abu, bb = w ? A.bbw : A.bbu;
-        const double gt = w ? A.gtw : A.gtu, gb = w ? A.gbw : A.gbu;
-        auto tt = [=](int n) -> double { return at + dy * bt * (double)n * (double)n; };
-        auto tb = [=](int n) -> double { double t = ab - dy * bb * (double)n * (double)n; return (n & 1) ? -t : t; };
-        PF un = tau_penta<NY>(r, A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, make_double2(gt, 0.0),
-                              make_double2(gb, 0.0), lane);
-        un = pf_real(un);
-        if (w == 0 && A.cmf) {
-          // constant mass flux: u0 += f phi, phi = response to a unit forcing
-          // held over the step (rhs -re/theta, homogeneous wall data)
-          PF unit = pf_zero<NY>();
-          if (lane == 0) unit.a[0] = make_double2(-A.re / th, 0.0);
-          PF phi = tau_penta<NY>(unit, A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-          phi = pf_real(phi);
-          const double bu = pf_bulk<NY>(un, lane), bp = pf_bulk<NY>(phi, lane);
-          const double fc = (A.ubulk - bu) / bp;
-          un = pf_axpy(fc, phi, un);
-          if (lane == 0) *A.dpdx = *A.dpdx - fc;
-        }
-        pf_store_real<NY>(um, lane, un);
-        pf_store_real<NY>(hl, lane, hcur);
-        pf_store_real<NY>(hn, lane, hcur);
-        if (w) w0p = un; else u0p = un;
-      }
-    }
-  } else {  // MODE 1 (startup): current state only
-    v = pf_load_pm<NY>(A.V, p, lane);
-    omy = pf_load_pm<NY>(A.OMY, p, lane);
-    if (is00) {
-      v = pf_zero<NY>(); omy = pf_zero<NY>();
-      pf_store_pm<NY>(A.V, p, lane, v);
-      pf_store_pm<NY>(A.OMY, p, lane, omy);
-      u0p = pf_load_real<NY>(A.u0, lane);
-      w0p = pf_load_real<NY>(A.w0, lane);
-    }
-  }
-
-  // ---------------- veloc / vort / gradscl (solvers.f90:1576-1722) ------
-  PF u, w;
-  if (is00) {
-    u = u0p;
-    w = w0p;
-  } else {
-    PF dv = cderiv<NY>(v, dy, lane);
-    const double ik2 = 1.0 / k2;
-    // u = -(-i kx Dv + i kz omy)/k2 ; w = -(-i kz Dv - i kx omy)/k2
-    u = pf_scale(pf_sub(pf_imul(dv, kx), pf_imul(omy, kz)), ik2);
-    w = pf_scale(pf_add(pf_imul(dv, kz), pf_imul(omy, kx)), ik2);
-  }
-  const PF du = cderiv<NY>(u, dy, lane), dw = cderiv<NY>(w, dy, lane);
-  PF ox = pf_sub(dw, pf_imul(v, kz));
-  PF oz = pf_sub(pf_imul(v, kx), du);
-  if (A.TPD[0]) {  // D u, D v, D w for the velocity-gradient tensor (gradv, derivatives.f90:6-86)
-    cheb_to_phys_store<NY, V>(du, buf, scr, twl, lane, static_cast<V*>(A.TPD[0]), P, p);
-    cheb_to_phys_store<NY, V>(cderiv<NY>(v, dy, lane), buf, scr, twl, lane, static_cast<V*>(A.TPD[1]), P, p);
-    cheb_to_phys_store<NY, V>(dw, buf, scr, twl, lane, static_cast<V*>(A.TPD[2]), P, p);
-  }
-  cheb_to_phys_store<NY, V>(u, buf, scr, twl, lane, TT[0], P, p);
-  cheb_to_phys_store<NY, V>(v, buf, scr, twl, lane, TT[1], P, p);
-  cheb_to_phys_store<NY, V>(w, buf, scr, twl, lane, TT[2], P, p);
-  cheb_to_phys_store<NY, V>(ox, buf, scr, twl, lane, TT[3], P, p);
-  cheb_to_phys_store<NY, V>(omy, buf, scr, twl, lane, TT[4], P, p);
-  cheb_to_phys_store<NY, V>(oz, buf, scr, twl, lane, TT[5], P, p);
-  if (SCALAR) {
-    PF tx = pf_imul(sc, kx), tz = pf_imul(sc, kz);
-    PF ty = cderiv<NY>(sc, dy, lane);
-    cheb_to_phys_store<NY, V>(tx, buf, scr, twl, lane, TT[6], P, p);
-    cheb_to_phys_store<NY, V>(ty, buf, scr, twl, lane, TT[7], P, p);
-    cheb_to_phys_store<NY, V>(tz, buf, scr, twl, lane, TT[8], P, p);
-  }
-}
-
-// The full step (MODE 0) with the [y][pencil] fields of the block (the
-// nonlinear terms in, the transfer fields out) staged through LDS tiles
-// (coalesced rows of PWS pencils); the state, stored pencil-major, is read
-// and written by each wave as contiguous memory.  Same operations in the
-// same order per pencil as pencil_body, so the results are identical; every
-// wave of the block, the z-Nyquist pencil's included, passes every block
-// barrier.
-template <int NY, bool SCALAR, typename V>
-__device__ __forceinline__ void pencil_step_tiled(const PencilArgs& A, int blk) {
-  using PF = PFN<NY>;
-  using G = TileG<NY>;
-  using LP = StepLds<NY, V, SCALAR>;
-  constexpr int NTS = LP::NTS;
-  extern __shared__ __align__(16) unsigned char smraw[];
-  V* smem = reinterpret_cast<V*>(smraw);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int p0 = blk * PWS, p = p0 + wv;
-  const V* twl = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
-  V* buf = smem + 2 * NY + (size_t)wv * FFTBuf<2 * NY>::len;
-  V* scr = buf;  // transforms in place
-  unsigned char* region = smraw + LP::TWB;
-  V* vtile = reinterpret_cast<V*>(region + LP::FFT);     // NL / transfer tiles after the FFT buffers
-  V* const* TT = reinterpret_cast<V* const*>(A.T);
-  const size_t P = (size_t)A.P;
-  const bool live = (size_t)p < P;
-  double kx, kz;
-  int kxi, kzi;
-  pencil_k(A, live ? p : 0, kx, kz, kxi, kzi);
-  const double k2 = kx * kx + kz * kz;
-  const bool is00 = live && kxi == 0 && kzi == 0;
-  const bool nyq = kzi == A.nzh;
-  const bool act = live && !nyq;  // computes; the z-Nyquist pencil is zeroed (helpers.f90:149-156)
-  const double dy = A.dyde;
-  const double th = A.theta;
-  // ---------------- part B: nonlinear terms -> fn, gn, scn (spectral) --
-  PF fn, gn, sn;
-  PF h1m, h3m;  // mean-mode profiles (only used by the (0,0) pencil)
-  if (A.first_nl) {
-    V r2[2][G::PER];
     {
-      V rn[2][G::PER];
-      tile_fetch<NY, V>(static_cast<const V*>(A.NL1), P, p0, rn[0]);
-      tile_fetch<NY, V>(static_cast<const V*>(A.NL3), P, p0, rn[1]);
-      tile_fetch<NY, V>(static_cast<const V*>(A.NL2), P, p0, r2[0]);
-      if (SCALAR) tile_fetch<NY, V>(static_cast<const V*>(A.NLS), P, p0, r2[1]);
-      tile_put<NY, V>(vtile, rn[0]);
-      tile_put<NY, V>(vtile + G::LEN, rn[1]);
-    }
-    __syncthreads();
-    PF h1, h3, h2;
-    if (act) {
-      h1 = phys_to_cheb<NY, V>(tile_phys<NY, V>(vtile, wv, lane), buf, scr, twl, lane);
-      h3 = phys_to_cheb<NY, V>(tile_phys<NY, V>(vtile + G::LEN, wv, lane), buf, scr, twl, lane);
-    }
-    __syncthreads();
-    tile_put<NY, V>(vtile, r2[0]);
-    if (SCALAR) tile_put<NY, V>(vtile + G::LEN, r2[1]);
-    __syncthreads();
-    if (act) {
-      const double sz = A.smooth ? A.smz[kzi] : 1.0;
-      h2 = phys_to_cheb<NY, V>(tile_phys<NY, V>(vtile, wv, lane), buf, scr, twl, lane);
-      if (A.TF[0]) {  // polymer force, subforce (helpers.f90:564-606), before smoothing
-        h1 = pf_add(h1, pf_load<NY>(A.TF[0], P, p, lane));
-        h2 = pf_add(h2, pf_load<NY>(A.TF[1], P, p, lane));
-        h3 = pf_add(h3, pf_load<NY>(A.TF[2], P, p, lane));
+      RD qg;
+      pm_fetch<NY>(qg, A.GNM1, p0, lane);
+      if (is00) omy = mean_load<NY>(A.u0, A.w0, l);
+      PF rhs = r_cderiv<NY>(r_cderiv<NY>(omy, dy, l), dy, l);
+      PF old = pm_take<NY>(qg, wd, lane);
+      rp_mask(old, nyq);
+      if (is00) {
+        old = mean_load<NY>(A.h1nm1, A.h3nm1, l);
+        mean_store<NY>(A.h1nm1, A.h3nm1, gn, l);
+        mean_store<NY>(A.h1n, A.h3n, gn, l);
       }
-      if (A.smooth) {
-        h1 = smooth_apply<NY>(h1, A.smy, sz, lane);
-        h2 = smooth_apply<NY>(h2, A.smy, sz, lane);
-        h3 = smooth_apply<NY>(h3, A.smy, sz, lane);
+      rhs = r_phirhs(omy, rhs, gn, old, k2, A.re, 1.0, A.dt, th);
+      rp_mask(gn, is00);
+      pm_store<NY>(A.GNM1, p0, wd, lane, gn);
+      double2 be = czero(), bo = czero();
+      if (is00) {
+        be = make_double2(0.5 * (A.gtu + A.gbu), 0.5 * (A.gtw + A.gbw));
+        bo = make_double2(0.5 * (A.gtu - A.gbu), 0.5 * (A.gtw - A.gbw));
       }
-      if (is00) { h1 = pf_real(h1); h2 = pf_real(h2); h3 = pf_real(h3); }
-      h1m = h1;
-      h3m = h3;
-      // nonlin (solvers.f90:1497-1572)
-      PF x = pf_add(pf_imul(h3, kz), pf_imul(h1, kx));
-      PF dx = cderiv<NY>(x, dy, lane);
-      fn = pf_sub(pf_scale(h2, -k2), dx);
-      gn = pf_sub(pf_imul(h1, kz), pf_imul(h3, kx));
-      if (SCALAR) {
-        sn = phys_to_cheb<NY, V>(tile_phys<NY, V>(vtile + G::LEN, wv, lane), buf, scr, twl, lane);
-        if (A.smooth) sn = smooth_apply<NY>(sn, A.smy, sz, lane);
-        if (is00) sn = pf_real(sn);
-      }
-    }
-    __syncthreads();  // the NL tiles become transfer tiles
-  } else {
-    if (act) {
-      fn = pf_load_pm<NY>(A.FN, p, lane);
-      gn = pf_load_pm<NY>(A.GN, p, lane);
-      if (SCALAR) sn = pf_load_pm<NY>(A.SCN, p, lane);
-      if (is00) { h1m = pf_load_real<NY>(A.h1n, lane); h3m = pf_load_real<NY>(A.h3n, lane); }
-    }
-  }
-
-  // ---------------- solves ----------------------------------------------
-  // The state is stored pencil-major: each wave loads its pencils
-  // (contiguous) where the solves use them, which keeps the kernel within
-  // the registers of three waves per SIMD.
-  PF sc, v, omy;
-  PF u0p, w0p;
-  if (act) {
-    // scalar (main_dns.f90:324-358)
-    if (SCALAR) {
-      sc = pf_load_pm<NY>(A.TH, p, lane);
-      const PF scnm1 = pf_load_pm<NY>(A.SCNM1, p, lane);
-      PF d1 = cderiv<NY>(sc, dy, lane);
-      PF d2 = cderiv<NY>(d1, dy, lane);
-      PF rhs = phirhs<NY>(sc, d2, sn, scnm1, k2, A.re, A.diff, A.dt, th);
-      pf_store_pm<NY>(A.SCNM1, p, lane, sn);
-      auto tt = [dy](int n) -> double { return dy * (double)n * (double)n; };
-      auto tb = [dy](int n) -> double { double v = dy * (double)n * (double)n; return (n & 1) ? -v : v; };
-      sc = tau_penta<NY>(rhs, k2 + A.gS, dy, A.tabS + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-      if (is00) sc = pf_real(sc);
-      pf_store_pm<NY>(A.TH, p, lane, sc);
-    }
-    // v and omega_y (main_dns.f90:360-502)
-    if (!is00) {
-      v = pf_load_pm<NY>(A.V, p, lane);
-      const PF fnm1 = pf_load_pm<NY>(A.FNM1, p, lane);
-      PF d1 = cderiv<NY>(v, dy, lane);
-      PF d2 = cderiv<NY>(d1, dy, lane);
-      PF phi = pf_sub(d2, pf_scale(v, k2));
-      d1 = cderiv<NY>(phi, dy, lane);
-      d2 = cderiv<NY>(d1, dy, lane);
-      PF rhs = phirhs<NY>(phi, d2, fn, fnm1, k2, A.re, 1.0, A.dt, th);
-      pf_store_pm<NY>(A.FNM1, p, lane, fn);
-      phi = tau_solve<NY>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p * tab_width(NY), czero(), czero(), 0, lane);
-      PF vp = tau_solve<NY>(phi, k2, dy, A.tabP + (size_t)p * tab_width(NY), czero(), czero(), 0, lane);
-      double2 vt, vb;
-      wall_derivs<NY>(vp, dy, lane, vt, vb);
-      const double4 g = A.gk[p];
-      double2 c1 = cadd(cscale(vb, g.x), cscale(vt, g.y));
-      double2 c2 = cadd(cscale(vb, g.z), cscale(vt, g.w));
-      v = pf_add(vp, pf_add(pf_cmul_real(c1, green_load<NY>(A.G1, p, lane)),
-                            pf_cmul_real(c2, green_load<NY>(A.G2, p, lane))));
-      omy = pf_load_pm<NY>(A.OMY, p, lane);
-      const PF gnm1 = pf_load_pm<NY>(A.GNM1, p, lane);
-      PF e1 = cderiv<NY>(omy, dy, lane);
-      PF e2 = cderiv<NY>(e1, dy, lane);
-      PF orhs = phirhs<NY>(omy, e2, gn, gnm1, k2, A.re, 1.0, A.dt, th);
-      pf_store_pm<NY>(A.GNM1, p, lane, gn);
-      const double atu = A.atu, btu = A.btu, abu = A.abu, bbu = A.bbu;
-      auto tt = [=](int n) -> double { return atu + dy * btu * (double)n * (double)n; };
-      auto tb = [=](int n) -> double { double t = abu + dy * bbu * (double)n * (double)n; return (n & 1) ? -t : t; };
-      omy = tau_penta<NY>(orhs, k2 + A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-      pf_store_pm<NY>(A.V, p, lane, v);
-      pf_store_pm<NY>(A.OMY, p, lane, omy);
-    } else {
-      // (0,0): v = 0 (veloc), omega_y = 0, fnm1 = fn = 0, gnm1 = gn = 0,
-      // and the mean-flow solves (uzero, solvers.f90:1065-1176).
-      v = pf_zero<NY>();
-      omy = pf_zero<NY>();
-      pf_store_pm<NY>(A.V, p, lane, v);
-      pf_store_pm<NY>(A.OMY, p, lane, omy);
-      pf_store_pm<NY>(A.FNM1, p, lane, pf_zero<NY>());
-      pf_store_pm<NY>(A.GNM1, p, lane, pf_zero<NY>());
-      for (int w = 0; w < 2; ++w) {
-        double* um = w ? A.w0 : A.u0;
-        double* hl = w ? A.h3nm1 : A.h1nm1;
-        double* hn = w ? A.h3n : A.h1n;
-        const PF& hcur = w ? h3m : h1m;
-        PF u = pf_load_real<NY>(um, lane);
-        PF hlp = pf_load_real<NY>(hl, lane);
-        PF d1 = cderiv<NY>(u, dy, lane);
-        PF d2 = cderiv<NY>(d1, dy, lane);
-        PF r = pf_scale(u, -A.re / (A.dt * th));
-        r = pf_axpy(-3.0 * A.re / (2.0 * th), hcur, r);
-        r = pf_axpy(A.re / (2.0 * th), hlp, r);
-        r = pf_axpy(-(1.0 - th) / th, d2, r);
-        const double at = w ? A.atw : A.atu, bt = A.btu, ab = w ? A.abw : A.abu, bb = w ? A.bbw : A.bbu;
-        const double gt = w ? A.gtw : A.gtu, gb = w ? A.gbw : A.gbu;
-        auto tt = [=](int n) -> double { return at + dy * bt * (double)n * (double)n; };
-        auto tb = [=](int n) -> double { double t = ab - dy * bb * (double)n * (double)n; return (n & 1) ? -t : t; };
-        PF un = tau_penta<NY>(r, A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, make_double2(gt, 0.0),
-                              make_double2(gb, 0.0), lane);
-        un = pf_real(un);
-        if (w == 0 && A.cmf) {
-          PF unit = pf_zero<NY>();
-          if (lane == 0) unit.a[0] = make_double2(-A.re / th, 0.0);
-          PF phi = tau_penta<NY>(unit, A.gH, dy, A.tabH + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-          phi = pf_real(phi);
-          const double bu = pf_bulk<NY>(un, lane), bp = pf_bulk<NY>(phi, lane);
-          const double fc = (A.ubulk - bu) / bp;
-          un = pf_axpy(fc, phi, un);
-          if (lane == 0) *A.dpdx = *A.dpdx - fc;
+      omy = r_solve<NY, false>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p0 * TW, rt, be, bo, l);
+      if (A.cmf && p0 == 0) {
+        // constant mass flux: u0 += f phi, phi = the response to a unit
+        // forcing held over the step (rhs -re/theta, homogeneous wall data)
+        rhs = rp_zero<NY>();
+        if (l == 0) rhs.a[0] = make_double2(-A.re / th, 0.0);
+        rhs = r_solve<NY, false>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p0 * TW, rt, czero(), czero(), l);
+        const double fc = (A.ubulk - r_bulk<NY>(omy, l)) / r_bulk<NY>(rhs, l);
+        if (is00) {
+          omy = pf_axpy(fc, rhs, omy);
+          if (l == 0) *A.dpdx = *A.dpdx - fc;
         }
-        pf_store_real<NY>(um, lane, un);
-        pf_store_real<NY>(hl, lane, hcur);
-        pf_store_real<NY>(hn, lane, hcur);
-        if (w) w0p = un; else u0p = un;
       }
+      if (is00) mean_store<NY>(A.u0, A.w0, omy, l);
+      rp_mask(omy, is00);
+      pm_store<NY>(A.OMY, p0, wd, lane, omy);
     }
-  } else if (live) {  // the z-Nyquist pencil: zero state
-    const PF z = pf_zero<NY>();
-    pf_store_pm<NY>(A.V, p, lane, z);
-    pf_store_pm<NY>(A.OMY, p, lane, z);
-    pf_store_pm<NY>(A.FNM1, p, lane, z);
-    pf_store_pm<NY>(A.GNM1, p, lane, z);
-    if (SCALAR) {
-      pf_store_pm<NY>(A.TH, p, lane, z);
-      pf_store_pm<NY>(A.SCNM1, p, lane, z);
+    RD qf;
+    v = pm_load<NY>(A.V, p0, wd, lane);
+    pm_fetch<NY>(qf, A.FNM1, p0, lane);
+    rp_mask(v, nyq || is00);
+    v = pf_axpy(-k2, v, r_cderiv<NY>(r_cderiv<NY>(v, dy, l), dy, l));  // phi
+    {
+      const PF d = r_cderiv<NY>(r_cderiv<NY>(v, dy, l), dy, l);
+      PF old = pm_take<NY>(qf, wd, lane);
+      rp_mask(old, nyq || is00);
+      v = r_phirhs(v, d, fn, old, k2, A.re, 1.0, A.dt, th);
     }
+    pm_store<NY>(A.FNM1, p0, wd, lane, fn);
+#pragma unroll 1
+    for (int s = 0; s < 2; ++s)  // phi, then v with homogeneous walls
+      v = r_solve<NY, false>(v, s ? k2 : k2 + A.gH, dy, (s ? A.tabP : A.tabH) + (size_t)p0 * TW, rt, czero(), czero(), l);
+    // influence matrix (main_dns.f90:433-466)
+    double2 vt, vb;
+    r_wall_derivs<NY>(v, dy, l, vt, vb);
+    const double4 g = (A.gk + p0)[row];
+    constexpr unsigned GW = NY / 2 + 1;
+    green_add<NY>(v, cadd(cscale(vb, g.x), cscale(vt, g.y)), A.G1 + (size_t)p0 * GW, row * GW, l);
+    green_add<NY>(v, cadd(cscale(vb, g.z), cscale(vt, g.w)), A.G2 + (size_t)p0 * GW, row * GW, l);
+    rp_mask(v, is00 || nyq);
+    pm_store<NY>(A.V, p0, wd, lane, v);
+  } else {  // startup: the current state, its (0,0) pencils zeroed
+    v = pm_load<NY>(A.V, p0, wd, lane);
+    if (p0 == 0) {
+      rp_mask(v, is00);
+      pm_store<NY>(A.V, p0, wd, lane, v);
+      PF o = pm_load<NY>(A.OMY, p0, wd, lane);
+      rp_mask(o, is00);
+      pm_store<NY>(A.OMY, p0, wd, lane, o);
+    }
+    rp_mask(v, is00 || nyq);
   }
 
-  // ---------------- veloc / vort / gradscl (solvers.f90:1576-1722) ------
-  PF u, w;
-  if (act) {
-    if (is00) {
-      u = u0p;
-      w = w0p;
-    } else {
-      PF dv = cderiv<NY>(v, dy, lane);
-      const double ik2 = 1.0 / k2;
-      u = pf_scale(pf_sub(pf_imul(dv, kx), pf_imul(omy, kz)), ik2);
-      w = pf_scale(pf_add(pf_imul(dv, kz), pf_imul(omy, kx)), ik2);
-    }
-  }
-  // inverse transforms into transfer tiles, NTS at a time; out(j) is the
-  // j-th transfer field, dst(j) its destination
-  auto flush = [&](int j0, int n, V* const* dst) {
-    __syncthreads();
-    for (int j = 0; j < n; ++j) tile_store<NY, V>(vtile + (size_t)j * G::LEN, dst[j0 + j], P, p0);
-    __syncthreads();
-  };
-  if (A.TPD[0]) {  // D u, D v, D w for the velocity-gradient tensor (gradv, derivatives.f90:6-86)
-    V* const D[3] = {static_cast<V*>(A.TPD[0]), static_cast<V*>(A.TPD[1]), static_cast<V*>(A.TPD[2])};
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      V* t = vtile + (size_t)j * G::LEN;
-      if (act) {
-        const PF d = cderiv<NY>(j == 0 ? u : (j == 1 ? v : w), dy, lane);
-        cheb_to_phys_tile<NY, V>(d, buf, scr, twl, lane, t, wv);
-      } else if (live) {
-        tile_col_zero<NY, V>(t, wv, lane);
+  // ---------------- veloc / vort (solvers.f90:1576-1722) ---------------
+  // D u, D v, D w (TPD) only for the velocity-gradient tensor (gradv,
+  // derivatives.f90:6-86)
+  PF d;
+  const double ik2 = 1.0 / k2;
+#pragma unroll 1
+  for (int j = 0; j < 9; ++j) {
+    PF o;
+    V* dst;
+    switch (j) {
+      case 0: o = v; dst = TT[1]; break;
+      case 1: o = omy; dst = TT[4]; break;
+      case 2: o = r_cderiv<NY>(v, dy, l); dst = TPD[1]; break;
+      case 3: case 6: {  // u, w
+        const PF dv = r_cderiv<NY>(v, dy, l);
+        o = pf_scale(pf_add(pf_imul(dv, j == 3 ? kx : kz), pf_imul(omy, j == 3 ? -kz : kx)), ik2);
+        if (is00) {
+          const PF m = mean_load<NY>(A.u0, A.w0, l);
+          o = j == 3 ? m : pf_imul(m, -1.0);
+          rp_mask_imag(o, true);
+        }
+        d = r_cderiv<NY>(o, dy, l);
+        dst = TT[j == 3 ? 0 : 2];
+        break;
       }
+      case 4: o = d; dst = TPD[0]; break;
+      case 5: o = pf_sub(pf_imul(v, kx), d); dst = TT[5]; break;  // omega_z
+      case 7: o = d; dst = TPD[2]; break;
+      default: o = pf_sub(d, pf_imul(v, kz)); dst = TT[3]; break;  // omega_x
     }
-    flush(0, 3, D);
-  }
-  // each transfer field is formed just before its transform, and
-  // D u, D w right after u, w leave: at most five pencil fields stay live
-  PF du, dw;
-  constexpr int NOUT = LP::NOUT;
-#pragma unroll
-  for (int j = 0; j < NOUT; ++j) {
-    V* t = vtile + (size_t)(j % NTS) * G::LEN;
-    if (act) {
-      PF o;
-      if (j == 0) o = u;
-      else if (j == 1) o = v;
-      else if (j == 2) o = w;
-      else if (j == 3) o = pf_sub(dw, pf_imul(v, kz));  // omega_x
-      else if (j == 4) o = omy;
-      else if (j == 5) o = pf_sub(pf_imul(v, kx), du);  // omega_z
-      else if (j == 6) o = pf_imul(sc, kx);
-      else if (j == 7) o = cderiv<NY>(sc, dy, lane);
-      else o = pf_imul(sc, kz);
-      cheb_to_phys_tile<NY, V>(o, buf, scr, twl, lane, t, wv);
-      if (j == 0) du = cderiv<NY>(u, dy, lane);
-      if (j == 2) dw = cderiv<NY>(w, dy, lane);
-    } else if (live) {
-      tile_col_zero<NY, V>(t, wv, lane);
-    }
-    if (j % NTS == NTS - 1 || j == NOUT - 1) flush(j - j % NTS, j % NTS + 1, TT);
+    if (dst) cheb_to_rows<NY, V>(o, w, tw, lane, dst, P, p0);
   }
 }
 
+// TV: occupancy variant picked by the autotuner (0: row_waves, 1: one instead
+// of two wavefronts per SIMD and two instead of one; 128 x 129 x 128 FP64 0.122
+// and 0.151 ms)
 template <int NY, bool SCALAR, int MODE, typename V, int TV = 0>
-__global__ __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3 : 1))) void k_pencil(PencilArgs A) {
-  if constexpr (MODE == 0 && StepLds<NY, V, SCALAR>::ok)
-    pencil_step_tiled<NY, SCALAR, V>(A, xcd_group(blockIdx.x, gridDim.x));
-  else pencil_body<NY, SCALAR, MODE, V>(A, blockIdx.x);
+__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3 - row_waves<NY>() : row_waves<NY>()))) void k_pencil(PencilArgs A) {
+  pencil_body<NY, SCALAR, MODE, V>(A, xcd_group(blockIdx.x, gridDim.x));
 }
 
 // The step kernel of an ensemble of channels of one size in one launch:
 // channel blockIdx.y takes its arguments from AA[blockIdx.y].
 template <int NY, bool SCALAR, typename V, int TV>
-__global__ __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3 : 1)))
+__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3 - row_waves<NY>() : row_waves<NY>())))
 void k_pencil_batch(const PencilArgs* __restrict__ AA) {
-  if constexpr (StepLds<NY, V, SCALAR>::ok)
-    pencil_step_tiled<NY, SCALAR, V>(AA[blockIdx.y], xcd_group(blockIdx.x, gridDim.x));
-  else pencil_body<NY, SCALAR, 0, V>(AA[blockIdx.y], blockIdx.x);
+  pencil_body<NY, SCALAR, 0, V>(AA[blockIdx.y], xcd_group(blockIdx.x, gridDim.x));
 }
 
 // -------------------------------------------------- parity kernels --
@@ -823,18 +535,20 @@ hipError_t launch_green(int ny, const PencilArgs& a, double pb1, double pt1, dou
                                           pt2, G1, G2, gk));
   return hipGetLastError();
 }
+// pencils come in blocks of 16 (nx/2 is a multiple of 8, nz even), the walls'
+// rows are Dirichlet rows of weight 1
+static bool row_ok(const PencilArgs& a) {
+  return a.P % (RWV * RPW) == 0 && a.nz % RPW == 0 && a.atu == 1.0 && a.abu == 1.0 && a.atw == 1.0 && a.abw == 1.0 &&
+         a.btu == 0.0 && a.bbu == 0.0 && a.btw == 0.0 && a.bbw == 0.0;
+}
 template <int MODE, typename V, int TV>
 static hipError_t launch_pencil_tv(int ny, const PencilArgs& a, hipStream_t s) {
+  if (!row_ok(a)) return hipErrorInvalidValue;
+  const dim3 grid(a.P / (RWV * RPW)), block(RWV * 64);
   if (a.scalar) {
-    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil<NY, true, MODE, V, TV>),
-                                           dim3(step_blocks<NY, V, true, MODE>(a.P)),
-                                           dim3(step_threads<NY, V, true, MODE>()),
-                                           (step_lds_bytes<NY, V, true, MODE>()), s, a));
+    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil<NY, true, MODE, V, TV>), grid, block, (row_lds<NY, V>()), s, a));
   } else {
-    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil<NY, false, MODE, V, TV>),
-                                           dim3(step_blocks<NY, V, false, MODE>(a.P)),
-                                           dim3(step_threads<NY, V, false, MODE>()),
-                                           (step_lds_bytes<NY, V, false, MODE>()), s, a));
+    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil<NY, false, MODE, V, TV>), grid, block, (row_lds<NY, V>()), s, a));
   }
   return hipGetLastError();
 }
@@ -853,16 +567,12 @@ hipError_t launch_pencil_step(int ny, const PencilArgs& a, hipStream_t s) { retu
 template <typename V, int TV>
 static hipError_t launch_pencil_batch_v(int ny, const PencilArgs& a0, const PencilArgs* dA, int nmem,
                                         hipStream_t s) {
+  if (!row_ok(a0)) return hipErrorInvalidValue;
+  const dim3 grid(a0.P / (RWV * RPW), nmem), block(RWV * 64);
   if (a0.scalar) {
-    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_batch<NY, true, V, TV>),
-                                           dim3(step_blocks<NY, V, true, 0>(a0.P), nmem),
-                                           dim3(step_threads<NY, V, true, 0>()),
-                                           (step_lds_bytes<NY, V, true, 0>()), s, dA));
+    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_batch<NY, true, V, TV>), grid, block, (row_lds<NY, V>()), s, dA));
   } else {
-    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_batch<NY, false, V, TV>),
-                                           dim3(step_blocks<NY, V, false, 0>(a0.P), nmem),
-                                           dim3(step_threads<NY, V, false, 0>()),
-                                           (step_lds_bytes<NY, V, false, 0>()), s, dA));
+    KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_batch<NY, false, V, TV>), grid, block, (row_lds<NY, V>()), s, dA));
   }
   return hipGetLastError();
 }

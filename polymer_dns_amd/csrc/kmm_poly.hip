@@ -98,9 +98,9 @@ __global__ __launch_bounds__(poly_pw<NY>() * 64) void k_poly_pencil(PolyArgs A) 
       }
       if (is00) { t1 = pf_real(t1); t2 = pf_real(t2); t3 = pf_real(t3); }
     }
-    pf_store<NY>(A.TF[0], P, p, lane, t1);
-    pf_store<NY>(A.TF[1], P, p, lane, t2);
-    pf_store<NY>(A.TF[2], P, p, lane, t3);
+    pf_store_pm<NY>(A.TF[0], p, lane, t1);
+    pf_store_pm<NY>(A.TF[1], p, lane, t2);
+    pf_store_pm<NY>(A.TF[2], p, lane, t3);
     return;
   }
   if (kzi == A.nzh) {  // norm zeroes the z-Nyquist row (helpers.f90:149-156)
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(poly_pw<NY>() * 64) void k_poly_pencil(PolyArgs A) 
         }
     }
     if (A.force && (MODE == 2 || A.partB))
-      for (int t = 0; t < 3; ++t) pf_store<NY>(A.TF[t], P, p, lane, z);
+      for (int t = 0; t < 3; ++t) pf_store_pm<NY>(A.TF[t], p, lane, z);
     return;
   }
 
@@ -208,9 +208,9 @@ __global__ __launch_bounds__(poly_pw<NY>() * 64) void k_poly_pencil(PolyArgs A) 
   }
   if (A.force && ((MODE == 0 && A.partB) || MODE == 2)) {
     if (is00) { t1 = pf_real(t1); t2 = pf_real(t2); t3 = pf_real(t3); }
-    pf_store<NY>(A.TF[0], P, p, lane, t1);
-    pf_store<NY>(A.TF[1], P, p, lane, t2);
-    pf_store<NY>(A.TF[2], P, p, lane, t3);
+    pf_store_pm<NY>(A.TF[0], p, lane, t1);
+    pf_store_pm<NY>(A.TF[1], p, lane, t2);
+    pf_store_pm<NY>(A.TF[2], p, lane, t3);
   }
 }
 

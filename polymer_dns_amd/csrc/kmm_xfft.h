@@ -32,7 +32,7 @@ namespace kmm {
 
 // ------------------------------------------------------- register DFTs --
 // dft<R>: R-point transform in registers, natural order, from the radix 2 to
-// 8 butterflies: coprime factors A B (12 = 3 4, 18 = 2 9, 24 = 3 8) by the
+// 8 butterflies: coprime factors A B (10 = 2 5, 12 = 3 4, 18 = 2 9, 24 = 3 8) by the
 // Good-Thomas index maps (n = B a + A b mod AB in, k = k mod A, k mod B out:
 // no twiddles), 9 and 16 as squares with constant twiddles.
 template <int DIR, typename V>
@@ -78,8 +78,10 @@ __device__ __forceinline__ void dft(V (&v)[R]) {
   if constexpr (R == 2) dft2<DIR>(v[0], v[1]);
   else if constexpr (R == 3) dft3<DIR>(v[0], v[1], v[2]);
   else if constexpr (R == 4) dft4<DIR>(v[0], v[1], v[2], v[3]);
+  else if constexpr (R == 5) dft5<DIR>(v[0], v[1], v[2], v[3], v[4]);
   else if constexpr (R == 6) dft_coprime<2, 3, DIR, V>(v);
   else if constexpr (R == 8) dft8<DIR>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]);
+  else if constexpr (R == 10) dft_coprime<2, 5, DIR, V>(v);
   else if constexpr (R == 12) dft_coprime<3, 4, DIR, V>(v);
   else if constexpr (R == 18) dft_coprime<2, 9, DIR, V>(v);
   else if constexpr (R == 24) dft_coprime<3, 8, DIR, V>(v);
