@@ -1,6 +1,6 @@
 // Pencil stage of the FENE-P conformation tensor (POLYMER build of the
-// reference), one wavefront per (kx,kz) pencil, the six independent
-// components c11, c12, c13, c22, c23, c33 one after another:
+// reference), four (kx,kz) pencils per wavefront (kmm_row.h), the six
+// independent components one after another:
 //
 //   part B  forward Chebyshev transform of the plane stage's c_n and str_n
 //           (solvers.f90:3279-3416); the polymer force
@@ -18,207 +18,206 @@
 //           y-derivatives, derivatives.f90:148-254; the x and z derivatives
 //           are taken in the plane stage).
 //
-// The conformation tensor and its histories (C, CN, CNM1, STRN, STRNM1) are
+// The conformation tensor, its histories (C, CNM1, ...) and the force TF are
 // stored pencil-major, [pencil][y] (the reference's order of a spectral
-// field): a wave reads and writes its pencil as contiguous memory.  The
-// fields shared with the plane stage (the physical-y NLP and TP fields, the
-// force TF) keep the [y][pencil] layout of the transforms.
+// field).  The fields shared with the plane stage (the physical-y NLP and TP
+// fields) keep the [y][pencil] layout of the transforms.
 //
 // MODE 0: step, MODE 1: startup (evaluate only), MODE 2: finish (part B only),
 // MODE 3: C from the physical-y fields in NLP[0..5] (a conformation tensor
 // rebuilt on the 3/2 grid and forward transformed in x and z), MODE 4: part B
 // of a learned-closure stress (the force only: a closure stress is neither
-// smoothed nor stored, and there is no conformation to transport), MODE 5:
-// the step after a separate MODE 2 pass (C init, solve and evaluate, reading
-// the smoothed c_n and str_n that pass stored; at ny = 192 the two passes
-// hold fewer registers than the fused step).
+// smoothed nor stored, and there is no conformation to transport).
 #include "kmm_kernels.h"
 #include "kmm_pencil.h"
+#include "kmm_row.h"
 
 namespace kmm {
 
-// Pencils (wavefronts) per workgroup. At ny = 192 the two-segment solve needs
-// more than 256 registers a lane: a 4-wave workgroup lets the compiler hold
-// them in the unified VGPR/AGPR file at one wave per SIMD instead of spilling
-// about 300 bytes a lane to scratch at two (4.5 % faster in FP64).
-template <int NY> constexpr int poly_pw() { return NY > 128 ? 4 : PW; }
+// A force component that waits for its other terms is held in LDS where two
+// wavefronts share a SIMD's registers, and in registers where one has them.
+template <int NY> constexpr bool poly_park() { return row_waves<NY>() > 1; }
+template <int NY, typename V>
+constexpr size_t poly_lds() {
+  return row_lds<NY, V>() + (poly_park<NY>() ? (size_t)RWV * 64 * (2 * RLay<NY>::K + 1) * sizeof(double2) : 0);
+}
+template <int NY>
+struct Parked {
+  RP<NY> r;
+  double2* q;
+  __device__ __forceinline__ void put(const RP<NY>& f) {
+    constexpr int K = RLay<NY>::K;
+    if (!poly_park<NY>()) { r = f; return; }
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      q[64 * 2 * i] = f.a[i];
+      q[64 * (2 * i + 1)] = f.b[i];
+    }
+    q[64 * 2 * K] = f.e;
+  }
+  __device__ __forceinline__ RP<NY> get() const {
+    constexpr int K = RLay<NY>::K;
+    if (!poly_park<NY>()) return r;
+    RP<NY> f;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      f.a[i] = q[64 * 2 * i];
+      f.b[i] = q[64 * (2 * i + 1)];
+    }
+    f.e = q[64 * 2 * K];
+    return f;
+  }
+};
 
+// The components run in the order 11, 12, 22, 23, 33, 13: two force
+// components are open at a time (t1 until 13; t2 until 23, then t3), and each
+// is stored as soon as it is complete, so that the registers hold one force,
+// the component's two terms and, in the solve, C and the right-hand side.
+//
+// Bound by memory: a step reads 30 and writes 45 fields of 16 B a coefficient
+// (2.85 GB at 192 x 129 x 192 FP64, 0.6 ms at the 4.8 TB/s of a large copy).
+// Measured against one pencil a wavefront: 192 x 129 x 192 FP64 1.13 -> 0.87
+// ms, mixed 0.98 -> 0.72 ms; 256 x 193 x 256 FP64, before in two passes of
+// fewer registers each, 4.00 -> 1.83 ms.
 template <int NY, int MODE, typename V>
-__global__ __launch_bounds__(poly_pw<NY>() * 64) void k_poly_pencil(PolyArgs A) {
-  using PF = PFN<NY>;
-  constexpr bool M0 = (MODE == 0 || MODE == 5);  // mode 5: mode 0 without part B
+__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
+void k_poly_pencil(PolyArgs A) {
+  using RL = RLay<NY>;
+  using PF = RP<NY>;
   extern __shared__ __align__(16) unsigned char smraw[];
   V* smem = reinterpret_cast<V*>(smraw);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int p = blockIdx.x * poly_pw<NY>() + wv;
-  const V* twl = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
-  if (p >= A.P) return;
-  V* buf = wave_lds<NY, V>(smem, wv);
-  V* scr = buf + FFTBuf<2 * NY>::len;
-  const size_t P = (size_t)A.P;
+  const V* tw = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
+  const int lane = threadIdx.x & 63, l = lane & 15, row = lane >> 4;
+  const unsigned wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double2* wd = reinterpret_cast<double2*>(smraw + 2 * NY * sizeof(V)) + (size_t)wv * RPW * RL::BUF;
+  V* w = reinterpret_cast<V*>(wd);
+  const unsigned P = (unsigned)A.P, p0 = (unsigned)(xcd_group(blockIdx.x, gridDim.x) * RWV + wv) * RPW;
+  constexpr unsigned TW = tab_width(NY);
   double kx, kz;
   int kxi, kzi;
-  pencil_k(A, p, kx, kz, kxi, kzi);
+  pencil_k(A, (int)p0 + row, kx, kz, kxi, kzi);
   const double k2 = kx * kx + kz * kz;
-  const bool is00 = (kxi == 0 && kzi == 0);
+  const bool is00 = (kxi == 0 && kzi == 0), nyq = (kzi == A.nzh);  // norm zeroes the z-Nyquist row
   const double dy = A.dyde;
-
-  if (MODE == 3) {
-#pragma unroll 1
-    for (int c = 0; c < 6; ++c) {
-      PF C = pf_zero<NY>();
-      if (kzi != A.nzh) {
-        C = phys_to_cheb_load<NY, V>(static_cast<const V*>(A.NLP[c]), P, p, buf, scr, twl, lane);
-        if (is00) C = pf_real(C);
-      }
-      pf_store_pm<NY>(A.C[c], p, lane, C);
-    }
-    return;
-  }
-  if (MODE == 4) {
-    // each component's load is issued before the previous one's transform
-    PF t1 = pf_zero<NY>(), t2 = pf_zero<NY>(), t3 = pf_zero<NY>();
-    if (kzi != A.nzh) {
-      PhysN<NY, V> q = phys_load<NY, V>(static_cast<const V*>(A.NLP[6]), P, p, lane);
-#pragma unroll 1
-      for (int c = 0; c < 6; ++c) {
-        const PhysN<NY, V> cur = q;
-        if (c < 5) q = phys_load<NY, V>(static_cast<const V*>(A.NLP[7 + c]), P, p, lane);
-        PF sn = phys_to_cheb<NY, V>(cur, buf, scr, twl, lane);
-        if (is00) sn = pf_real(sn);
-        const PF f = pf_scale(sn, A.zbeta1);
-        switch (c) {
-          case 0: t1 = pf_add(t1, pf_imul(f, kx)); break;
-          case 1: t1 = pf_add(t1, cderiv<NY>(f, dy, lane)); t2 = pf_add(t2, pf_imul(f, kx)); break;
-          case 2: t1 = pf_add(t1, pf_imul(f, kz)); t3 = pf_add(t3, pf_imul(f, kx)); break;
-          case 3: t2 = pf_add(t2, cderiv<NY>(f, dy, lane)); break;
-          case 4: t2 = pf_add(t2, pf_imul(f, kz)); t3 = pf_add(t3, cderiv<NY>(f, dy, lane)); break;
-          default: t3 = pf_add(t3, pf_imul(f, kz)); break;
-        }
-      }
-      if (is00) { t1 = pf_real(t1); t2 = pf_real(t2); t3 = pf_real(t3); }
-    }
-    pf_store_pm<NY>(A.TF[0], p, lane, t1);
-    pf_store_pm<NY>(A.TF[1], p, lane, t2);
-    pf_store_pm<NY>(A.TF[2], p, lane, t3);
-    return;
-  }
-  if (kzi == A.nzh) {  // norm zeroes the z-Nyquist row (helpers.f90:149-156)
-    const PF z = pf_zero<NY>();
-    for (int c = 0; c < 6; ++c) {
-      if (M0 || MODE == 2) {
-        if (A.partB || MODE == 2) {
-          if (!A.closure) pf_store_pm<NY>(A.CN[c], p, lane, z);
-          if (!A.closure || MODE == 2) pf_store_pm<NY>(A.STRN[c], p, lane, z);
-        }
-        if (A.copy || A.solve) { pf_store_pm<NY>(A.CNM1[c], p, lane, z); pf_store_pm<NY>(A.STRNM1[c], p, lane, z); }
-      }
-      if (M0 && (A.init || A.solve)) pf_store_pm<NY>(A.C[c], p, lane, z);
-      if (MODE != 2 && A.evaluate)
-        for (int h = 0; h < 2; ++h) {
-          pf_store_zero<NY, V>(static_cast<V*>(A.TP[c + 6 * h]), P, p, lane);
-        }
-    }
-    if (A.force && (MODE == 2 || A.partB))
-      for (int t = 0; t < 3; ++t) pf_store_pm<NY>(A.TF[t], p, lane, z);
-    return;
-  }
-
   const double sz = A.smooth ? A.smz[kzi] : 1.0;
   const double ti = 1.0 / A.tpoly;
-  PF t1 = pf_zero<NY>(), t2 = pf_zero<NY>(), t3 = pf_zero<NY>();
+  const bool haveB = MODE == 2 || MODE == 4 || (MODE == 0 && A.partB);
+  const bool force = MODE == 4 || (A.force && haveB);
+  auto term = [&](const void* F) -> PF {
+    RowRaw<NY, V> q;
+    rows_fetch<NY, V>(q, static_cast<const V*>(F), P, p0, lane);
+    PF h = rows_to_cheb<NY, V>(q, w, tw, lane);
+    rp_mask_imag(h, is00);
+    rp_mask(h, nyq);
+    return h;
+  };
+  auto load = [&](const double2* F) -> PF {
+    PF h = pm_load<NY>(F, p0, wd, lane);
+    rp_mask(h, nyq);
+    return h;
+  };
+  PF tA = rp_zero<NY>();
+  Parked<NY> tB;
+  tB.q = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + (size_t)wv * 64 * (2 * RL::K + 1) + lane;
 #pragma unroll 1
-  for (int c = 0; c < 6; ++c) {
-    // component c: 11, 12, 13, 22, 23, 33
+  for (int it = 0; it < 6; ++it) {
+    const int c = (0x254310 >> (4 * it)) & 7;  // components 11, 12, 13, 22, 23, 33 as 0..5
+    if (MODE == 3) {
+      pm_store<NY>(A.C[c], p0, wd, lane, term(A.NLP[c]));
+      continue;
+    }
     PF cn, sn;
-    PF cnm1_copy, snm1_copy;
-    const bool haveB = (MODE == 2) || (MODE == 0 && A.partB);
     if (haveB) {
-      cn = A.closure ? pf_zero<NY>() : phys_to_cheb_load<NY, V>(static_cast<const V*>(A.NLP[c]), P, p, buf, scr, twl, lane);
-      sn = phys_to_cheb_load<NY, V>(static_cast<const V*>(A.NLP[6 + c]), P, p, buf, scr, twl, lane);
-      if (is00) { cn = pf_real(cn); sn = pf_real(sn); }
-      if (A.force) {
+      sn = term(A.NLP[6 + c]);
+      if (force) {
         // t_i = d q_ik / d x_k with q = zbeta1 str (symmetric)
-        const PF q = pf_scale(sn, A.zbeta1);
-        switch (c) {
-          case 0: t1 = pf_add(t1, pf_imul(q, kx)); break;
-          case 1: t1 = pf_add(t1, cderiv<NY>(q, dy, lane)); t2 = pf_add(t2, pf_imul(q, kx)); break;
-          case 2: t1 = pf_add(t1, pf_imul(q, kz)); t3 = pf_add(t3, pf_imul(q, kx)); break;
-          case 3: t2 = pf_add(t2, cderiv<NY>(q, dy, lane)); break;
-          case 4: t2 = pf_add(t2, pf_imul(q, kz)); t3 = pf_add(t3, cderiv<NY>(q, dy, lane)); break;
-          default: t3 = pf_add(t3, pf_imul(q, kz)); break;
+        const double z = A.zbeta1, zx = z * kx, zz = z * kz;
+        PF d = sn;
+        if (c == 1 || c == 3 || c == 4) d = r_cderiv<NY>(sn, z * dy, l);
+        if (c < 3) tA = pf_add(tA, c == 1 ? d : pf_imul(sn, c == 0 ? zx : zz));
+        if (c == 2) {
+          rp_mask_imag(tA, is00);
+          pm_store<NY>(A.TF[0], p0, wd, lane, tA);
+        }
+        if (c != 0) {
+          PF t = c == 3 ? d : pf_imul(sn, c < 3 ? zx : zz);
+          if (c != 1) t = pf_add(t, tB.get());
+          if (c == 2 || c == 4) {
+            rp_mask_imag(t, is00);
+            pm_store<NY>(A.TF[c == 2 ? 2 : 1], p0, wd, lane, t);
+            t = d;
+          }
+          tB.put(t);
         }
       }
+      if (MODE == 4) continue;
+      cn = rp_zero<NY>();
+      if (!A.closure) cn = term(A.NLP[c]);
       if (A.copy) {
-        cnm1_copy = cn;
-        snm1_copy = sn;
-        pf_store_pm<NY>(A.CNM1[c], p, lane, cn);
-        pf_store_pm<NY>(A.STRNM1[c], p, lane, sn);
+        pm_store<NY>(A.CNM1[c], p0, wd, lane, cn);
+        pm_store<NY>(A.STRNM1[c], p0, wd, lane, sn);
+        // the solve below reads them back through other lanes
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
       }
       // a closure stress feeds only the force: in a step its smoothed copy
       // in STRN has no reader (an explicit finish still stores it)
       const bool keep = !A.closure || MODE == 2;
       if (A.smooth && keep) {
-        cn = smooth_apply<NY>(cn, A.smy, sz, lane);
-        sn = smooth_apply<NY>(sn, A.smy, sz, lane);
+        r_smooth<NY>(cn, A.smy, sz, l);
+        r_smooth<NY>(sn, A.smy, sz, l);
       }
-      if (!A.closure) pf_store_pm<NY>(A.CN[c], p, lane, cn);
-      if (keep) pf_store_pm<NY>(A.STRN[c], p, lane, sn);
+      if (!A.closure) pm_store<NY>(A.CN[c], p0, wd, lane, cn);
+      if (keep) pm_store<NY>(A.STRN[c], p0, wd, lane, sn);
       if (MODE == 2) continue;
     }
     PF C;
-    if (M0) {
-      if (A.init) {
-        C = pf_zero<NY>();
-        if (is00 && (c == 0 || c == 3 || c == 5)) {
-          const double v0 = A.c0[c == 0 ? 0 : (c == 3 ? 1 : 2)];
-          if (lane == 0) C.a[0] = make_double2(v0, 0.0);
-        }
-      } else {
-        C = pf_load_pm<NY>(A.C[c], p, lane);
+    if (MODE == 0 && A.solve) {
+      // cNL = 3 (c_n - str_n/lambda) - (c_nm1 - str_nm1/lambda)
+      if (!haveB) {
+        cn = load(A.CN[c]);
+        sn = load(A.STRN[c]);
       }
-      if (A.solve) {
-        if (!haveB) {
-          cn = pf_load_pm<NY>(A.CN[c], p, lane);
-          sn = pf_load_pm<NY>(A.STRN[c], p, lane);
-        }
-        const PF cm = A.copy && haveB ? cnm1_copy : pf_load_pm<NY>(A.CNM1[c], p, lane);
-        const PF sm = A.copy && haveB ? snm1_copy : pf_load_pm<NY>(A.STRNM1[c], p, lane);
-        // cNL = 3 (c_n - str_n/lambda) - (c_nm1 - str_nm1/lambda)
-        const PF nl = pf_sub(pf_scale(pf_axpy(-ti, sn, cn), 3.0), pf_axpy(-ti, sm, cm));
-        pf_store_pm<NY>(A.CNM1[c], p, lane, cn);
-        pf_store_pm<NY>(A.STRNM1[c], p, lane, sn);
-        const PF d1 = cderiv<NY>(C, dy, lane);
-        const PF d2 = cderiv<NY>(d1, dy, lane);
-        const PF rhs = phirhs<NY>(C, d2, nl, pf_scale(nl, 2.0), k2, A.re, A.diffpoly, A.dt, A.theta);
-        // Neumann rows at both walls (at = ab = 0, bt = bb = 1, zero data)
-        auto tt = [dy](int n) -> double { return dy * (double)n * (double)n; };
-        auto tb = [dy](int n) -> double { double v = dy * (double)n * (double)n; return (n & 1) ? -v : v; };
-        C = tau_penta<NY>(rhs, k2 + A.gC, dy, A.tabC + (size_t)p * tab_width(NY), tt, tb, czero(), czero(), lane);
-        if (is00) C = pf_real(C);
+      {
+        PF old = load(A.CNM1[c]);
+        pm_store<NY>(A.CNM1[c], p0, wd, lane, cn);
+        cn = pf_sub(pf_scale(pf_axpy(-ti, sn, cn), 3.0), old);
+        old = load(A.STRNM1[c]);
+        pm_store<NY>(A.STRNM1[c], p0, wd, lane, sn);
+        cn = pf_axpy(ti, old, cn);
       }
-      if (A.init || A.solve) pf_store_pm<NY>(A.C[c], p, lane, C);
+    }
+    if (MODE == 0 && A.init) {
+      C = rp_zero<NY>();
+      if (is00 && l == 0 && (c == 0 || c == 3 || c == 5)) C.a[0] = make_double2(A.c0[c == 0 ? 0 : (c == 3 ? 1 : 2)], 0.0);
     } else {
-      C = pf_load_pm<NY>(A.C[c], p, lane);
+      C = load(A.C[c]);
     }
+    if (MODE == 0 && A.solve) {
+      // phirhs with fn = cNL, fnm1 = 2 cNL: 3 fn - fnm1 = cNL; Neumann rows
+      const double c0 = -A.re * A.diffpoly / (A.dt * A.theta), c2 = (1.0 - A.theta) / A.theta;
+      cn = pf_axpy(-A.re * A.diffpoly / (2.0 * A.theta), cn, pf_scale(C, c0 + c2 * k2));
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) C = r_cderiv<NY>(C, dy, l);
+      C = pf_axpy(-c2, C, cn);
+      C = r_solve<NY, true>(C, k2 + A.gC, dy, A.tabC + (size_t)p0 * TW, row * TW, czero(), czero(), l);
+      rp_mask_imag(C, is00);
+    }
+    if (MODE == 0 && (A.init || A.solve)) pm_store<NY>(A.C[c], p0, wd, lane, C);
     if (A.evaluate) {
-      cheb_to_phys_store<NY, V>(C, buf, scr, twl, lane, static_cast<V*>(A.TP[c]), P, p);
-      cheb_to_phys_store<NY, V>(cderiv<NY>(C, dy, lane), buf, scr, twl, lane, static_cast<V*>(A.TP[6 + c]), P, p);
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        cheb_to_rows<NY, V>(C, w, tw, lane, static_cast<V*>(A.TP[c + 6 * h]), P, p0);
+        if (h == 0) C = r_cderiv<NY>(C, dy, l);
+      }
     }
-  }
-  if (A.force && ((MODE == 0 && A.partB) || MODE == 2)) {
-    if (is00) { t1 = pf_real(t1); t2 = pf_real(t2); t3 = pf_real(t3); }
-    pf_store_pm<NY>(A.TF[0], p, lane, t1);
-    pf_store_pm<NY>(A.TF[1], p, lane, t2);
-    pf_store_pm<NY>(A.TF[2], p, lane, t3);
   }
 }
 
 template <int MODE, typename V>
 static hipError_t launch_poly_v(int ny, const PolyArgs& a, hipStream_t s) {
-  KMM_NY_DISPATCH(ny, constexpr int W = poly_pw<NY>();
-                  hipLaunchKernelGGL((k_poly_pencil<NY, MODE, V>), dim3((a.P + W - 1) / W), dim3(W * 64),
-                                     (lds_bytes<NY, V>(W)), s, a));
+  if (a.P % (RWV * RPW) != 0 || a.nz % RPW != 0) return hipErrorInvalidValue;
+  KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_poly_pencil<NY, MODE, V>), dim3(a.P / (RWV * RPW)), dim3(RWV * 64),
+                                         (poly_lds<NY, V>()), s, a));
   return hipGetLastError();
 }
 
@@ -229,7 +228,6 @@ hipError_t launch_poly_pencil(int ny, int mode, const PolyArgs& a, bool mixed, h
     case 2: return mixed ? launch_poly_v<2, float2>(ny, a, s) : launch_poly_v<2, double2>(ny, a, s);
     case 3: return mixed ? launch_poly_v<3, float2>(ny, a, s) : launch_poly_v<3, double2>(ny, a, s);
     case 4: return mixed ? launch_poly_v<4, float2>(ny, a, s) : launch_poly_v<4, double2>(ny, a, s);
-    case 5: return mixed ? launch_poly_v<5, float2>(ny, a, s) : launch_poly_v<5, double2>(ny, a, s);
     default: return hipErrorInvalidValue;
   }
 }
