@@ -131,6 +131,7 @@ struct kmm_ctx {
   float* capg = nullptr;                          // [9][Pphys] du_i/dx_k of the last evaluation
   int hist_n = 0, hist_it = -1000;                // consecutive captured evaluations, last one
   kmm_mlp* closure = nullptr;                     // network replacing the conformation transport
+  bool cn_in_nm1 = false;  // the last step's terms are in CNM1, STRNM1 only: CN, STRN are older
   bool nlp_closure = false;                       // NLP holds only a closure stress (no c_n)
   // audits of the closure: windows of full FENE-P transport every audit_every
   // steps, restarted from C rebuilt from the closure's stress
@@ -1221,11 +1222,24 @@ static int materialize(kmm_ctx* c) {
     pa.closure = c->nlp_closure ? 1 : 0;
     int r = run_poly_pencil(c, 2, pa);
     if (r) return r;
+    if (!pa.closure) c->cn_in_nm1 = false;
     if (c->pprev.force) for (int q = 0; q < 3; ++q) a.TF[q] = c->TF[q];
   }
   hipError_t e = kmm::launch_pencil_finish(c->ny, a, c->stream);
   if (e != hipSuccess) return fail(KMM_E_HIP, std::string("pencil finish: ") + hipGetErrorString(e));
   KMM_HIP(hipStreamSynchronize(c->stream));
+  return KMM_OK;
+}
+
+// CN, STRN as a step leaves them, for a caller that drops the evaluation
+// which would replace them.
+static int own_cn(kmm_ctx* c) {
+  if (!c->cn_in_nm1) return KMM_OK;
+  for (int q = 0; q < 6; ++q) {
+    KMM_HIP(hipMemcpyAsync(c->CN[q], c->CNM1[q], c->S * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
+    KMM_HIP(hipMemcpyAsync(c->STRN[q], c->STRNM1[q], c->S * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
+  }
+  c->cn_in_nm1 = false;
   return KMM_OK;
 }
 
@@ -1303,6 +1317,7 @@ extern "C" int kmm_startup(kmm_ctx* c) {
       KMM_HIP(hipMemcpyAsync(c->STRNM1[q], c->STRN[q], c->S * sizeof(double2), hipMemcpyDeviceToDevice, c->stream));
     }
   }
+  c->cn_in_nm1 = false;
   c->pprev = pf;
   const size_t fb = c->S * sizeof(double2);
   KMM_HIP(hipMemcpyAsync(c->FNM1, c->FN, fb, hipMemcpyDeviceToDevice, c->stream));
@@ -1381,6 +1396,7 @@ static int enqueue_step(kmm_ctx* c, int s, hipEvent_t* ev, bool stage_ev) {
     const bool force_only = clo && pa.partB && pa.closure && pa.force && !pa.copy;
     const int r = run_poly_pencil(c, force_only ? 4 : 0, pa);
     if (r) return r;
+    if (pa.partB && !pa.closure) c->cn_in_nm1 = pa.solve;
     if (pa.force) for (int q = 0; q < 3; ++q) a.TF[q] = c->TF[q];
   }
   if (pf.evaluate && !clo) for (int q = 0; q < 3; ++q) a.TPD[q] = c->TPD[q];  // D u_i for the FENE-P plane
@@ -1526,6 +1542,7 @@ static int step_chunk_enqueue(kmm_ctx* c, int remaining, StepChunk& ch) {
       if (c->closure) c->hist_it = itsave;
     }
     KMM_HIP(hipGraphLaunch(c->gexec, c->stream));
+    if (c->cfg.polymer && !c->nlp_closure && c->pprev.solve) c->cn_in_nm1 = true;
     if (c->closure)
       for (int q = 1; q <= n; ++q) hist_note(c, c->it + q);
     c->it += n;
@@ -1835,6 +1852,8 @@ extern "C" int kmm_read_restart(kmm_ctx* c, const char* path) {
   std::vector<double> buf(6 * fs + 6 * ms, 0.0);
   for (int q = 0; q < 6; ++q) std::copy(rec.begin() + q * fsf, rec.begin() + (q + 1) * fsf, buf.begin() + q * fs);
   std::copy(rec.begin() + 6 * fsf, rec.end(), buf.begin() + 6 * fs);
+  int r0 = own_cn(c);
+  if (r0) return r0;
   c->nl_valid = false;
   const int ids[6] = {KMM_V, KMM_FN, KMM_FNM1, KMM_OMY, KMM_GN, KMM_GNM1};
   for (int q = 0; q < 6; ++q) {
@@ -2362,6 +2381,7 @@ static int vcw3dp_body(kmm_ctx* c, const double* u, const double* v, const doubl
       for (size_t e = 0; e < 2 * c->S; ++e) poly->qp[q][e] = zb * poly->strn[q][e];
     }
   }
+  if ((r = own_cn(c))) return r;
   c->nl_valid = false;
   return check_cfl(c, 1, it);
 }

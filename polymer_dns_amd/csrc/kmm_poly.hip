@@ -74,11 +74,15 @@ struct Parked {
 // is stored as soon as it is complete, so that the registers hold one force,
 // the component's two terms and, in the solve, C and the right-hand side.
 //
-// Bound by memory: a step reads 30 and writes 45 fields of 16 B a coefficient
-// (2.85 GB at 192 x 129 x 192 FP64, 0.6 ms at the 4.8 TB/s of a large copy).
-// Measured against one pencil a wavefront: 192 x 129 x 192 FP64 1.13 -> 0.87
-// ms, mixed 0.98 -> 0.72 ms; 256 x 193 x 256 FP64, before in two passes of
-// fewer registers each, 4.00 -> 1.83 ms.
+// Bound by memory: a step reads 30 and writes 33 fields of 16 B a coefficient
+// (2.4 GB at 192 x 129 x 192 FP64, 0.5 ms at the 4.8 TB/s of a large copy).
+// Measured against one pencil a wavefront with CN and STRN stored as well (12
+// fields more): 192 x 129 x 192 FP64 1.13 -> 0.74 ms (0.87 with them), mixed
+// 0.98 -> 0.61 ms; 256 x 193 x 256 FP64, before in two passes of fewer
+// registers each, 4.00 -> 1.60 ms (1.83 with them).  At ny = 128 one
+// wavefront a SIMD with every value in registers is the same (0.71, mixed
+// 0.64) and at ny = 64 slower (256 x 65 x 128 0.27 against 0.38 ms); loads
+// issued a component ahead gave nothing at either.
 template <int NY, int MODE, typename V>
 __global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
 void k_poly_pencil(PolyArgs A) {
@@ -166,8 +170,11 @@ void k_poly_pencil(PolyArgs A) {
         r_smooth<NY>(cn, A.smy, sz, l);
         r_smooth<NY>(sn, A.smy, sz, l);
       }
-      if (!A.closure) pm_store<NY>(A.CN[c], p0, wd, lane, cn);
-      if (keep) pm_store<NY>(A.STRN[c], p0, wd, lane, sn);
+      // a solve stores them below as the next step's n-1 terms
+      if (MODE == 2 || !A.solve) {
+        if (!A.closure) pm_store<NY>(A.CN[c], p0, wd, lane, cn);
+        if (keep) pm_store<NY>(A.STRN[c], p0, wd, lane, sn);
+      }
       if (MODE == 2) continue;
     }
     PF C;
