@@ -240,10 +240,10 @@ struct MrArgs {
   const double* cap;        // u, v, w, swirl [4][P]
   const double* mrf;        // wx, wy, wz, du_i/dx_k [12][P]
   const double* lap;        // Laplacians [3][P]
-  const double* uold;       // u, v, w of the previous evaluation [3][P]; replaced by the
-                            // rates (u - u_old)/dt (dt = t.dt) before the integration
-  const double* lold;       // Laplacians of the previous evaluation [3][P]; replaced by
-                            // their rates likewise
+  const double* uold;       // u, v, w of the previous evaluation [3][P]; may be replaced by
+                            // the rates (u - u_old)/dt (dt = t.dt) before the integration
+  const double* lold;       // Laplacians of the previous evaluation [3][P]; may be replaced
+                            // by their rates likewise
   int substep, cd_switch, swirl;
   double re, ratio, c_mu, gravity, dtfull;
 };
