@@ -372,6 +372,212 @@ __global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3
   pencil_body<NY, SCALAR, MODE, V>(A, xcd_group(blockIdx.x, gridDim.x));
 }
 
+// The step with a block's four wavefronts on the same four pencils, where a
+// channel has too few pencils to fill the chip with a wavefront each:
+//   wavefront 0  h1; omega_y (and the mean flow); u, omega_z
+//   wavefront 1  h2; v; v, D v
+//   wavefront 2  h3; w, omega_x
+//   wavefront 3  the scalar, or phi and its derivatives for wavefront 1; omega_y
+// with a block barrier after the nonlinear terms and after the solves; what
+// passes between wavefronts stands in LDS as the lanes hold it.  Bound by the
+// chain of wavefront 1: one transform, two solves, the wall correction, two
+// transforms, against the whole step's in pencil_body.
+constexpr int kTeamFields = 5;  // h1, h3, omega_y, v (phi before), D^2 phi
+template <int NY, typename V>
+constexpr size_t team_lds() { return row_lds<NY, V>() + (size_t)kTeamFields * lane_slots<NY>() * sizeof(double2); }
+template <int NY, bool SCALAR, typename V>
+__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
+void k_pencil_team(PencilArgs A) {
+  using RL = RLay<NY>;
+  using PF = RP<NY>;
+  extern __shared__ __align__(16) unsigned char smraw[];
+  V* smem = reinterpret_cast<V*>(smraw);
+  const V* tw = lds_twiddles<NY, V>(smem, static_cast<const V*>(A.twM));
+  const int lane = threadIdx.x & 63, l = lane & 15, row = lane >> 4;
+  const unsigned wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double2* wd = reinterpret_cast<double2*>(smraw + 2 * NY * sizeof(V)) + (size_t)wv * RPW * RL::BUF;
+  V* w = reinterpret_cast<V*>(wd);
+  double2* X = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + lane;
+  double2 *XH1 = X, *XH3 = X + lane_slots<NY>(), *XO = X + 2 * lane_slots<NY>(), *XV = X + 3 * lane_slots<NY>(),
+          *XD = X + 4 * lane_slots<NY>();
+  const unsigned P = (unsigned)A.P, p0 = (unsigned)xcd_group(blockIdx.x, gridDim.x) * RPW;
+  constexpr unsigned TW = tab_width(NY);
+  const unsigned rt = row * TW;
+  V* const* TT = reinterpret_cast<V* const*>(A.T);
+  V* const* TPD = reinterpret_cast<V* const*>(A.TPD);
+  double kx, kz;
+  int kxi, kzi;
+  pencil_k(A, (int)p0 + row, kx, kz, kxi, kzi);
+  const double k2 = kx * kx + kz * kz;
+  const bool is00 = (kxi == 0 && kzi == 0), nyq = (kzi == A.nzh);
+  const double dy = A.dyde, th = A.theta;
+  const double sz = A.smooth ? A.smz[kzi] : 1.0;
+  auto load = [&](const double2* F) -> PF {
+    PF h = pm_load<NY>(F, p0, wd, lane);
+    rp_mask(h, nyq);
+    return h;
+  };
+  auto phi_parts = [&](PF& phi, PF& d) {
+    phi = pm_load<NY>(A.V, p0, wd, lane);
+    rp_mask(phi, nyq || is00);
+    phi = pf_axpy(-k2, phi, r_cderiv<NY>(r_cderiv<NY>(phi, dy, l), dy, l));
+    d = r_cderiv<NY>(r_cderiv<NY>(phi, dy, l), dy, l);
+  };
+
+  // nonlinear terms; a wavefront's own in h
+  PF h = rp_zero<NY>();
+  const bool scal = SCALAR && wv == 3;
+  if (A.first_nl && (wv < 3 || scal)) {
+    const void* F = wv == 0 ? A.NL1 : wv == 1 ? A.NL2 : wv == 2 ? A.NL3 : A.NLS;
+    RowRaw<NY, V> q;
+    rows_fetch<NY, V>(q, static_cast<const V*>(F), P, p0, lane);
+    h = rows_to_cheb<NY, V>(q, w, tw, lane);
+    if (wv < 3 && A.TF[wv]) h = pf_add(h, pm_load<NY>(A.TF[wv], p0, wd, lane));
+    if (A.smooth) r_smooth<NY>(h, A.smy, sz, l);
+    rp_mask_imag(h, is00);
+    rp_mask(h, nyq);
+    if (wv == 0) lane_put<NY>(XH1, h);
+    if (wv == 2) lane_put<NY>(XH3, h);
+  } else if (!SCALAR && wv == 3) {
+    PF d;
+    phi_parts(h, d);
+    lane_put<NY>(XV, h);
+    lane_put<NY>(XD, d);
+  }
+  __syncthreads();
+
+  if (wv == 0) {  // omega_y and the mean flow
+    PF gn;
+    if (A.first_nl) {
+      gn = is00 ? h : pf_imul(h, kz);
+      gn = pf_sub(gn, pf_imul(lane_get<NY>(XH3), is00 ? -1.0 : kx));
+    } else {
+      gn = load(A.GN);
+      if (is00) gn = mean_load<NY>(A.h1n, A.h3n, l);
+    }
+    PF omy = load(A.OMY);
+    rp_mask(omy, is00);
+    if (is00) omy = mean_load<NY>(A.u0, A.w0, l);
+    PF rhs = r_cderiv<NY>(r_cderiv<NY>(omy, dy, l), dy, l);
+    PF old = load(A.GNM1);
+    if (is00) {
+      old = mean_load<NY>(A.h1nm1, A.h3nm1, l);
+      mean_store<NY>(A.h1nm1, A.h3nm1, gn, l);
+      mean_store<NY>(A.h1n, A.h3n, gn, l);
+    }
+    rhs = r_phirhs(omy, rhs, gn, old, k2, A.re, 1.0, A.dt, th);
+    rp_mask(gn, is00);
+    pm_store<NY>(A.GNM1, p0, wd, lane, gn);
+    double2 be = czero(), bo = czero();
+    if (is00) {
+      be = make_double2(0.5 * (A.gtu + A.gbu), 0.5 * (A.gtw + A.gbw));
+      bo = make_double2(0.5 * (A.gtu - A.gbu), 0.5 * (A.gtw - A.gbw));
+    }
+    omy = r_solve<NY, false>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p0 * TW, rt, be, bo, l);
+    if (A.cmf && p0 == 0) {  // constant mass flux, as in pencil_body
+      rhs = rp_zero<NY>();
+      if (l == 0) rhs.a[0] = make_double2(-A.re / th, 0.0);
+      rhs = r_solve<NY, false>(rhs, k2 + A.gH, dy, A.tabH + (size_t)p0 * TW, rt, czero(), czero(), l);
+      const double fc = (A.ubulk - r_bulk<NY>(omy, l)) / r_bulk<NY>(rhs, l);
+      if (is00) {
+        omy = pf_axpy(fc, rhs, omy);
+        if (l == 0) *A.dpdx = *A.dpdx - fc;
+      }
+    }
+    if (is00) mean_store<NY>(A.u0, A.w0, omy, l);
+    rp_mask(omy, is00);
+    lane_put<NY>(XO, omy);
+    pm_store<NY>(A.OMY, p0, wd, lane, omy);
+  } else if (wv == 1) {  // phi, v
+    PF fn;
+    if (A.first_nl) {
+      fn = pf_add(pf_imul(lane_get<NY>(XH1), kx), pf_imul(lane_get<NY>(XH3), kz));
+      fn = pf_sub(pf_scale(h, -k2), r_cderiv<NY>(fn, dy, l));
+    } else {
+      fn = load(A.FN);
+    }
+    PF v, d;
+    if (SCALAR) {
+      phi_parts(v, d);
+    } else {
+      v = lane_get<NY>(XV);
+      d = lane_get<NY>(XD);
+    }
+    {
+      PF old = load(A.FNM1);
+      rp_mask(old, is00);
+      v = r_phirhs(v, d, fn, old, k2, A.re, 1.0, A.dt, th);
+    }
+    pm_store<NY>(A.FNM1, p0, wd, lane, fn);
+#pragma unroll 1
+    for (int s = 0; s < 2; ++s)  // phi, then v with homogeneous walls
+      v = r_solve<NY, false>(v, s ? k2 : k2 + A.gH, dy, (s ? A.tabP : A.tabH) + (size_t)p0 * TW, rt, czero(), czero(), l);
+    double2 vt, vb;
+    r_wall_derivs<NY>(v, dy, l, vt, vb);
+    const double4 g = (A.gk + p0)[row];
+    constexpr unsigned GW = NY / 2 + 1;
+    green_add<NY>(v, cadd(cscale(vb, g.x), cscale(vt, g.y)), A.G1 + (size_t)p0 * GW, row * GW, l);
+    green_add<NY>(v, cadd(cscale(vb, g.z), cscale(vt, g.w)), A.G2 + (size_t)p0 * GW, row * GW, l);
+    rp_mask(v, is00 || nyq);
+    lane_put<NY>(XV, v);
+    pm_store<NY>(A.V, p0, wd, lane, v);
+  } else if (scal) {
+    PF sn = h;
+    if (!A.first_nl) sn = load(A.SCN);
+    PF sc = load(A.TH);
+    PF rhs = r_cderiv<NY>(r_cderiv<NY>(sc, dy, l), dy, l);
+    PF old = load(A.SCNM1);
+    rhs = r_phirhs(sc, rhs, sn, old, k2, A.re, A.diff, A.dt, th);
+    pm_store<NY>(A.SCNM1, p0, wd, lane, sn);
+    sc = r_solve<NY, true>(rhs, k2 + A.gS, dy, A.tabS + (size_t)p0 * TW, rt, czero(), czero(), l);
+    rp_mask_imag(sc, is00);
+    pm_store<NY>(A.TH, p0, wd, lane, sc);
+#pragma unroll 1
+    for (int j = 0; j < 3; ++j) {
+      PF o = pf_imul(sc, j == 0 ? kx : kz);
+      if (j == 1) o = r_cderiv<NY>(sc, dy, l);
+      cheb_to_rows<NY, V>(o, w, tw, lane, TT[6 + j], P, p0);
+    }
+  }
+  __syncthreads();
+
+  // veloc / vort: wavefronts 0 and 2 u and w, their D, omega_z and omega_x;
+  // 1 v, D v; 3 omega_y
+  const PF v = lane_get<NY>(XV);
+  const bool uw = wv == 0 || wv == 2, isu = wv == 0;
+  PF o, d;
+  if (wv == 1) {
+    o = v;
+    d = r_cderiv<NY>(v, dy, l);
+  } else {
+    o = lane_get<NY>(XO);
+    if (uw) {
+      const double ik2 = 1.0 / k2;
+      o = pf_scale(pf_add(pf_imul(r_cderiv<NY>(v, dy, l), isu ? kx : kz), pf_imul(o, isu ? -kz : kx)), ik2);
+      if (is00) {
+        const PF m = mean_load<NY>(A.u0, A.w0, l);
+        o = isu ? m : pf_imul(m, -1.0);
+        rp_mask_imag(o, true);
+      }
+      d = r_cderiv<NY>(o, dy, l);
+    }
+  }
+#pragma unroll 1
+  for (int j = 0; j < 3; ++j) {
+    V* dst;
+    if (j == 0) {
+      dst = TT[wv == 3 ? 4 : wv];
+    } else if (j == 1) {
+      dst = wv == 3 ? nullptr : TPD[wv];
+      o = d;
+    } else {
+      dst = uw ? TT[isu ? 5 : 3] : nullptr;
+      o = isu ? pf_sub(pf_imul(v, kx), d) : pf_sub(d, pf_imul(v, kz));
+    }
+    if (dst) cheb_to_rows<NY, V>(o, w, tw, lane, dst, P, p0);
+  }
+}
+
 // The step kernel of an ensemble of channels of one size in one launch:
 // channel blockIdx.y takes its arguments from AA[blockIdx.y].
 template <int NY, bool SCALAR, typename V, int TV>
@@ -541,10 +747,27 @@ static bool row_ok(const PencilArgs& a) {
   return a.P % (RWV * RPW) == 0 && a.nz % RPW == 0 && a.atu == 1.0 && a.abu == 1.0 && a.atw == 1.0 && a.abw == 1.0 &&
          a.btu == 0.0 && a.bbu == 0.0 && a.btw == 0.0 && a.bbw == 0.0;
 }
+// Four wavefronts on the same pencils where that leaves the blocks one or two
+// rounds on the 256 CUs.  Measured, a wavefront per four pencils -> four (us):
+//   2048 pencils  ny 64 34 -> 19 (mixed with scalar 40 -> 22), 128 46 -> 38
+//                 (55 -> 44), 192 61 -> 51; 512 pencils, ny 32 27 -> 12.5
+//   4608 pencils  ny 48 40 -> 33 (FP64 with scalar 60 -> 48), 64 45 -> 36, 80
+//                 mixed with scalar 65 -> 63, 128 73 -> 93, 192 138 -> 133
+//   8192 pencils  ny 32 39 -> 43, 48 51 -> 55, 64 51 -> 57, 128 70 -> 143
+static bool team_ok(int ny, int P) { return P <= 2048 || (P <= 5120 && ny <= 64); }
 template <int MODE, typename V, int TV>
 static hipError_t launch_pencil_tv(int ny, const PencilArgs& a, hipStream_t s) {
   if (!row_ok(a)) return hipErrorInvalidValue;
   const dim3 grid(a.P / (RWV * RPW)), block(RWV * 64);
+  if (MODE == 0 && TV == 0 && team_ok(ny, a.P)) {
+    const dim3 tgrid(a.P / RPW);
+    if (a.scalar) {
+      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, true, V>), tgrid, block, (team_lds<NY, V>()), s, a));
+    } else {
+      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, false, V>), tgrid, block, (team_lds<NY, V>()), s, a));
+    }
+    return hipGetLastError();
+  }
   if (a.scalar) {
     KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil<NY, true, MODE, V, TV>), grid, block, (row_lds<NY, V>()), s, a));
   } else {

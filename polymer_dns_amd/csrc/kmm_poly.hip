@@ -39,34 +39,17 @@ namespace kmm {
 template <int NY> constexpr bool poly_park() { return row_waves<NY>() > 1; }
 template <int NY, typename V>
 constexpr size_t poly_lds() {
-  return row_lds<NY, V>() + (poly_park<NY>() ? (size_t)RWV * 64 * (2 * RLay<NY>::K + 1) * sizeof(double2) : 0);
+  return row_lds<NY, V>() + (poly_park<NY>() ? (size_t)RWV * lane_slots<NY>() * sizeof(double2) : 0);
 }
 template <int NY>
 struct Parked {
   RP<NY> r;
   double2* q;
   __device__ __forceinline__ void put(const RP<NY>& f) {
-    constexpr int K = RLay<NY>::K;
-    if (!poly_park<NY>()) { r = f; return; }
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      q[64 * 2 * i] = f.a[i];
-      q[64 * (2 * i + 1)] = f.b[i];
-    }
-    q[64 * 2 * K] = f.e;
+    if (poly_park<NY>()) lane_put<NY>(q, f);
+    else r = f;
   }
-  __device__ __forceinline__ RP<NY> get() const {
-    constexpr int K = RLay<NY>::K;
-    if (!poly_park<NY>()) return r;
-    RP<NY> f;
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      f.a[i] = q[64 * 2 * i];
-      f.b[i] = q[64 * (2 * i + 1)];
-    }
-    f.e = q[64 * 2 * K];
-    return f;
-  }
+  __device__ __forceinline__ RP<NY> get() const { return poly_park<NY>() ? lane_get<NY>(q) : r; }
 };
 
 // The components run in the order 11, 12, 22, 23, 33, 13: two force
@@ -122,7 +105,7 @@ void k_poly_pencil(PolyArgs A) {
   };
   PF tA = rp_zero<NY>();
   Parked<NY> tB;
-  tB.q = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + (size_t)wv * 64 * (2 * RL::K + 1) + lane;
+  tB.q = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + (size_t)wv * lane_slots<NY>() + lane;
 #pragma unroll 1
   for (int it = 0; it < 6; ++it) {
     const int c = (0x254310 >> (4 * it)) & 7;  // components 11, 12, 13, 22, 23, 33 as 0..5

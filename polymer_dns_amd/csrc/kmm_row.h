@@ -590,6 +590,30 @@ __device__ __forceinline__ void cheb_to_rows(const RP<NY>& f, V* w, const V* tw,
   row_fft<NY, V>(b, tw, l);
   rows_store<NY, V>(w, dst, P, p0, lane);
 }
+// a lane's values in LDS, as held (q: the field's [2 K + 1][64], from the lane on)
+template <int NY> constexpr int lane_slots() { return 64 * (2 * RLay<NY>::K + 1); }
+template <int NY>
+__device__ __forceinline__ void lane_put(double2* q, const RP<NY>& f) {
+  constexpr int K = RLay<NY>::K;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    q[64 * 2 * i] = f.a[i];
+    q[64 * (2 * i + 1)] = f.b[i];
+  }
+  q[64 * 2 * K] = f.e;
+}
+template <int NY>
+__device__ __forceinline__ RP<NY> lane_get(const double2* q) {
+  constexpr int K = RLay<NY>::K;
+  RP<NY> f;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    f.a[i] = q[64 * 2 * i];
+    f.b[i] = q[64 * (2 * i + 1)];
+  }
+  f.e = q[64 * 2 * K];
+  return f;
+}
 // real mean profiles u, w as the parts of one complex pencil
 template <int NY>
 __device__ __forceinline__ RP<NY> mean_load(const double* __restrict__ u, const double* __restrict__ w, int l) {
