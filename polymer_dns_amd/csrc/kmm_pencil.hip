@@ -378,13 +378,15 @@ __global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3
 //   wavefront 1  h2; v; v, D v
 //   wavefront 2  h3; w, omega_x
 //   wavefront 3  the scalar, or phi and its derivatives for wavefront 1; omega_y
-// with a block barrier after the nonlinear terms and after the solves; what
-// passes between wavefronts stands in LDS as the lanes hold it.  Bound by the
-// chain of wavefront 1: one transform, two solves, the wall correction, two
+// with block barriers after the nonlinear terms, after fn and gn have been
+// formed from them and after the solves; what passes between wavefronts stands
+// in LDS as the lanes hold it, omega_y and v in the place of h1 and h3 (at ny =
+// 128 that lets two blocks share a CU: 2048 pencils 38 -> 27 us).  Bound by
+// the chain of wavefront 1: one transform, two solves, the wall correction, two
 // transforms, against the whole step's in pencil_body.
-constexpr int kTeamFields = 5;  // h1, h3, omega_y, v (phi before), D^2 phi
-template <int NY, typename V>
-constexpr size_t team_lds() { return row_lds<NY, V>() + (size_t)kTeamFields * lane_slots<NY>() * sizeof(double2); }
+// h1, h3, then omega_y, v; without the scalar phi and D^2 phi beside them
+template <int NY, bool SCALAR, typename V>
+constexpr size_t team_lds() { return row_lds<NY, V>() + (SCALAR ? 2 : 4) * (size_t)lane_slots<NY>() * sizeof(double2); }
 template <int NY, bool SCALAR, typename V>
 __global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
 void k_pencil_team(PencilArgs A) {
@@ -398,8 +400,8 @@ void k_pencil_team(PencilArgs A) {
   double2* wd = reinterpret_cast<double2*>(smraw + 2 * NY * sizeof(V)) + (size_t)wv * RPW * RL::BUF;
   V* w = reinterpret_cast<V*>(wd);
   double2* X = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + lane;
-  double2 *XH1 = X, *XH3 = X + lane_slots<NY>(), *XO = X + 2 * lane_slots<NY>(), *XV = X + 3 * lane_slots<NY>(),
-          *XD = X + 4 * lane_slots<NY>();
+  double2 *XH1 = X, *XH3 = X + lane_slots<NY>(), *XP = X + 2 * lane_slots<NY>(), *XD = X + 3 * lane_slots<NY>();
+  double2 *const XO = XH1, *const XV = XH3;  // once these have been read
   const unsigned P = (unsigned)A.P, p0 = (unsigned)xcd_group(blockIdx.x, gridDim.x) * RPW;
   constexpr unsigned TW = tab_width(NY);
   const unsigned rt = row * TW;
@@ -441,17 +443,24 @@ void k_pencil_team(PencilArgs A) {
   } else if (!SCALAR && wv == 3) {
     PF d;
     phi_parts(h, d);
-    lane_put<NY>(XV, h);
+    lane_put<NY>(XP, h);
     lane_put<NY>(XD, d);
+  }
+  __syncthreads();
+  if (A.first_nl) {  // gn (the (0,0) pencil's: h1 + i h3) and fn from the terms
+    if (wv == 0) {
+      h = is00 ? h : pf_imul(h, kz);
+      h = pf_sub(h, pf_imul(lane_get<NY>(XH3), is00 ? -1.0 : kx));
+    } else if (wv == 1) {
+      const PF f = pf_add(pf_imul(lane_get<NY>(XH1), kx), pf_imul(lane_get<NY>(XH3), kz));
+      h = pf_sub(pf_scale(h, -k2), r_cderiv<NY>(f, dy, l));
+    }
   }
   __syncthreads();
 
   if (wv == 0) {  // omega_y and the mean flow
-    PF gn;
-    if (A.first_nl) {
-      gn = is00 ? h : pf_imul(h, kz);
-      gn = pf_sub(gn, pf_imul(lane_get<NY>(XH3), is00 ? -1.0 : kx));
-    } else {
+    PF gn = h;
+    if (!A.first_nl) {
       gn = load(A.GN);
       if (is00) gn = mean_load<NY>(A.h1n, A.h3n, l);
     }
@@ -489,18 +498,13 @@ void k_pencil_team(PencilArgs A) {
     lane_put<NY>(XO, omy);
     pm_store<NY>(A.OMY, p0, wd, lane, omy);
   } else if (wv == 1) {  // phi, v
-    PF fn;
-    if (A.first_nl) {
-      fn = pf_add(pf_imul(lane_get<NY>(XH1), kx), pf_imul(lane_get<NY>(XH3), kz));
-      fn = pf_sub(pf_scale(h, -k2), r_cderiv<NY>(fn, dy, l));
-    } else {
-      fn = load(A.FN);
-    }
+    PF fn = h;
+    if (!A.first_nl) fn = load(A.FN);
     PF v, d;
     if (SCALAR) {
       phi_parts(v, d);
     } else {
-      v = lane_get<NY>(XV);
+      v = lane_get<NY>(XP);
       d = lane_get<NY>(XD);
     }
     {
@@ -747,24 +751,26 @@ static bool row_ok(const PencilArgs& a) {
   return a.P % (RWV * RPW) == 0 && a.nz % RPW == 0 && a.atu == 1.0 && a.abu == 1.0 && a.atw == 1.0 && a.abw == 1.0 &&
          a.btu == 0.0 && a.bbu == 0.0 && a.btw == 0.0 && a.bbw == 0.0;
 }
-// Four wavefronts on the same pencils where that leaves the blocks one or two
+// Four wavefronts on the same pencils where that leaves the blocks about two
 // rounds on the 256 CUs.  Measured, a wavefront per four pencils -> four (us):
-//   2048 pencils  ny 64 34 -> 19 (mixed with scalar 40 -> 22), 128 46 -> 38
-//                 (55 -> 44), 192 61 -> 51; 512 pencils, ny 32 27 -> 12.5
+//   512 pencils   ny 32 27 -> 12.7
+//   2048 pencils  ny 64 34 -> 19 (mixed with scalar 40 -> 22), 128 46 -> 27
+//                 (55 -> 30), 192 61 -> 51
 //   4608 pencils  ny 48 40 -> 33 (FP64 with scalar 60 -> 48), 64 45 -> 36, 80
-//                 mixed with scalar 65 -> 63, 128 73 -> 93, 192 138 -> 133
-//   8192 pencils  ny 32 39 -> 43, 48 51 -> 55, 64 51 -> 57, 128 70 -> 143
-static bool team_ok(int ny, int P) { return P <= 2048 || (P <= 5120 && ny <= 64); }
+//                 mixed with scalar 66 -> 64, 128 73 -> 65, 192 138 -> 133
+//   8192 pencils  ny 32 39 -> 43, 48 51 -> 55, 64 51 -> 55, 128 mixed with
+//                 scalar 100 -> 123
+static bool team_ok(int P) { return P <= 5120; }
 template <int MODE, typename V, int TV>
 static hipError_t launch_pencil_tv(int ny, const PencilArgs& a, hipStream_t s) {
   if (!row_ok(a)) return hipErrorInvalidValue;
   const dim3 grid(a.P / (RWV * RPW)), block(RWV * 64);
-  if (MODE == 0 && TV == 0 && team_ok(ny, a.P)) {
+  if (MODE == 0 && TV == 0 && team_ok(a.P)) {
     const dim3 tgrid(a.P / RPW);
     if (a.scalar) {
-      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, true, V>), tgrid, block, (team_lds<NY, V>()), s, a));
+      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, true, V>), tgrid, block, (team_lds<NY, true, V>()), s, a));
     } else {
-      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, false, V>), tgrid, block, (team_lds<NY, V>()), s, a));
+      KMM_NY_DISPATCH(ny, hipLaunchKernelGGL((k_pencil_team<NY, false, V>), tgrid, block, (team_lds<NY, false, V>()), s, a));
     }
     return hipGetLastError();
   }
