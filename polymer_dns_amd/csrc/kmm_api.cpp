@@ -104,7 +104,7 @@ struct kmm_ctx {
   double* mrf = nullptr;                 // [12][P] vorticity, velocity gradient
   double* lap[2] = {nullptr, nullptr};   // [3][P] Laplacians, current / previous evaluation
   int lap_cur = 0;
-  double* uold = nullptr;                // [3][P] u, v, w of the previous evaluation
+  double* uold = nullptr;                // [4][P] u, v, w of the previous evaluation (and room for the swirl)
   void* lapT = nullptr;                  // [3] Laplacians in physical y (transfer precision)
   void* lapZ = nullptr;                  // [3] after the z inverse
   bool cap_valid = false;
@@ -1095,19 +1095,16 @@ static int mr_laplacians(kmm_ctx* c) {
   return KMM_OK;
 }
 
-// u, v, w and the Laplacians of this evaluation become the old ones of the
-// next (solvers.f90:3468-3474)
-static int mr_keep_old(kmm_ctx* c) {
-  const size_t P = (size_t)c->nyp * c->mz * c->mx;
-  KMM_HIP(hipMemcpyAsync(c->uold, c->cap, 3 * P * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-  c->lap_cur = 1 - c->lap_cur;
-  return KMM_OK;
-}
+// the Laplacians of this evaluation become the old ones of the next
+// (solvers.f90:3468-3474); u, v, w do so when that begins (run_plane)
+static void mr_keep_old(kmm_ctx* c) { c->lap_cur = 1 - c->lap_cur; }
 
 static int run_plane(kmm_ctx* c, int it, unsigned long long* cfl, hipEvent_t* ev = nullptr, bool track = false,
                      bool poly = false, bool closure = false) {
   PlaneArgs pa = plane_args(c, it, cfl);
   const bool trk = track && c->npart > 0;
+  // the physical u, v, w of the last evaluation are now the old ones
+  if (trk && inertial(c)) std::swap(c->cap, c->uold);
   if (trk) pa.cap = c->cap;
   if (blob_active(c, it)) {
     // solvers.f90:2078-2118 at the particle positions before this step's update
@@ -1177,7 +1174,7 @@ static int run_plane(kmm_ctx* c, int it, unsigned long long* cfl, hipEvent_t* ev
     m.dtfull = c->cfg.dt;
     if ((e = kmm::launch_inertial(m, c->stream)) != hipSuccess)
       return fail(KMM_E_HIP, std::string("inertial particles: ") + hipGetErrorString(e));
-    if ((r = mr_keep_old(c))) return r;
+    mr_keep_old(c);
     c->cap_valid = true;
   } else if (trk) {
     kmm::TracerArgs t = tracer_args(c);
@@ -1192,7 +1189,7 @@ static int run_plane(kmm_ctx* c, int it, unsigned long long* cfl, hipEvent_t* ev
     if (mr) {  // init_part of inertial particles: keep this evaluation's fields as the old ones
       int r = mr_laplacians(c);
       if (r) return r;
-      if ((r = mr_keep_old(c))) return r;
+      mr_keep_old(c);
     }
     c->part_state = 2;
     c->cap_valid = true;
@@ -2442,7 +2439,7 @@ static int mr_buffers(kmm_ctx* c) {
   const size_t P = (size_t)c->nyp * c->mz * c->mx;
   KMM_HIP(hipMalloc((void**)&c->mrf, 12 * P * sizeof(double)));
   for (int b = 0; b < 2; ++b) KMM_HIP(hipMalloc((void**)&c->lap[b], 3 * P * sizeof(double)));
-  KMM_HIP(hipMalloc((void**)&c->uold, 3 * P * sizeof(double)));
+  KMM_HIP(hipMalloc((void**)&c->uold, 4 * P * sizeof(double)));  // changes places with cap
   KMM_HIP(hipMalloc(&c->lapT, 3 * (size_t)c->nyp * c->nxh * c->nz * c->vsz));
   KMM_HIP(hipMalloc(&c->lapZ, 3 * (size_t)c->nyp * c->mz * c->nxh * c->vsz));
   c->lap_cur = 0;
