@@ -11,6 +11,10 @@
 // transforms (solvers.f90:2241-2546).  Projections of ``norm`` that couple
 // +kz and -kz are applied once per step in the plane stage (they commute
 // with every pencil operation); the pencil-local ones are applied here.
+// Products are contracted with additions within an expression only, so that
+// the step's two forms (a wavefront per four pencils, four wavefronts on them)
+// round alike whatever the compiler makes of their surroundings.
+#pragma clang fp contract(on)
 #include "kmm_kernels.h"
 #include "kmm_pencil.h"
 #include "kmm_row.h"
@@ -388,8 +392,7 @@ __global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(TV ? 3
 template <int NY, bool SCALAR, typename V>
 constexpr size_t team_lds() { return row_lds<NY, V>() + (SCALAR ? 2 : 4) * (size_t)lane_slots<NY>() * sizeof(double2); }
 template <int NY, bool SCALAR, typename V>
-__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
-void k_pencil_team(PencilArgs A) {
+__device__ __forceinline__ void team_body(const PencilArgs& A, int blk) {
   using RL = RLay<NY>;
   using PF = RP<NY>;
   extern __shared__ __align__(16) unsigned char smraw[];
@@ -402,7 +405,7 @@ void k_pencil_team(PencilArgs A) {
   double2* X = reinterpret_cast<double2*>(smraw + row_lds<NY, V>()) + lane;
   double2 *XH1 = X, *XH3 = X + lane_slots<NY>(), *XP = X + 2 * lane_slots<NY>(), *XD = X + 3 * lane_slots<NY>();
   double2 *const XO = XH1, *const XV = XH3;  // once these have been read
-  const unsigned P = (unsigned)A.P, p0 = (unsigned)xcd_group(blockIdx.x, gridDim.x) * RPW;
+  const unsigned P = (unsigned)A.P, p0 = (unsigned)blk * RPW;
   constexpr unsigned TW = tab_width(NY);
   const unsigned rt = row * TW;
   V* const* TT = reinterpret_cast<V* const*>(A.T);
@@ -580,6 +583,12 @@ void k_pencil_team(PencilArgs A) {
     }
     if (dst) cheb_to_rows<NY, V>(o, w, tw, lane, dst, P, p0);
   }
+}
+
+template <int NY, bool SCALAR, typename V>
+__global__ __launch_bounds__(RWV * 64) __attribute__((amdgpu_waves_per_eu(row_waves<NY>())))
+void k_pencil_team(PencilArgs A) {
+  team_body<NY, SCALAR, V>(A, xcd_group(blockIdx.x, gridDim.x));
 }
 
 // The step kernel of an ensemble of channels of one size in one launch:

@@ -35,10 +35,9 @@ def run(p, st, variant, **kw):
                                      (128, "scalar"), (192, "flow"), (192, "scalar")])
 @pytest.mark.parametrize("precision", [0, 1])
 def test_team_and_rows_agree(ny, kind, precision):
-    """The same operations in both forms, so FP64 differs by the compiler's
-    contraction only: 1e-12.  Mixed: a value that rounds to FP32 the other way
-    is 6e-8 of it, 1e-6 of the state; second derivatives in y magnify it in
-    the nonlinear terms as in the other step tests, 5e-3."""
+    """Bit for bit: the two forms write the same expressions, and products are
+    contracted with additions within an expression only.  (A member of an
+    ensemble, whose launches take the rows' form, equals the channel alone.)"""
     p = params(32, ny, 32, dt=0.002, scalar=kind == "scalar")
     st = seeded(p, 23, amp=0.2)
     if kind != "scalar":
@@ -54,7 +53,4 @@ def test_team_and_rows_agree(ny, kind, precision):
     print(f"case: step forms, 32 x {ny + 1} x 32, {kind}, precision {precision}", flush=True)
     a, b = run(p, st, 0, **kw), run(p, st, 1, **kw)
     for k in a:
-        e = rel(a[k], b[k])
-        derived = k in ("fn", "gn", "scn", "fnm1", "gnm1", "scnm1", "h1n", "h3n")
-        assert np.isfinite(a[k]).all()
-        assert e < (1e-12 if precision == 0 else 5e-3 if derived else 1e-6), (k, e)
+        assert np.isfinite(a[k]).all() and np.array_equal(a[k], b[k]), (k, rel(a[k], b[k]))
