@@ -160,8 +160,6 @@ __device__ __forceinline__ W suffix_affine_t(double c, W w, int lane) {
   const W yin = (row == 0) ? y1 : ((row == 1) ? y2 : y3);
   return affine_apply(c, w, yin);
 }
-__device__ __forceinline__ double2 suffix_affine(double c, double2 w, int lane) { return suffix_affine_t<double2>(c, w, lane); }
-__device__ __forceinline__ double suffix_affine_r(double c, double w, int lane) { return suffix_affine_t<double>(c, w, lane); }
 
 // Prefix affine recurrence y_l = a_l + b_l * y_{l-1} (y_{-1} = 0).
 __device__ __forceinline__ double2 prefix_affine(double b, double2 a, int lane) {

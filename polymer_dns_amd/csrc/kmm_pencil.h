@@ -88,15 +88,6 @@ __device__ __forceinline__ PFT<S> pf_real(const PFT<S>& x) {
   r.e.y = 0.0;
   return r;
 }
-// complex number times a real pencil coefficientwise
-template <int S>
-__device__ __forceinline__ PFT<S> pf_cmul_real(double2 c, const PFT<S>& g) {
-  PFT<S> r;
-#pragma unroll
-  for (int s = 0; s < S; ++s) { r.a[s] = cscale(c, g.a[s].x); r.b[s] = cscale(c, g.b[s].x); }
-  r.e = cscale(c, g.e.x);
-  return r;
-}
 
 // ------------------------------------------- cross-segment lane moves --
 // value of pair g+1 (0 past the last segment)
@@ -222,31 +213,6 @@ __device__ __forceinline__ PFN<NY> pf_load_pm(const double2* __restrict__ F, siz
   }
   f.e = f0[NY];
   return f;
-}
-template <int NY>
-__device__ __forceinline__ void pf_store_pm(double2* __restrict__ F, size_t p, int lane, const PFN<NY>& f) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-  double2* f0 = F + p * (size_t)(NY + 1);
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g = s * WAVE + lane;
-    if (g < L) {
-      f0[2 * g] = f.a[s];
-      f0[2 * g + 1] = f.b[s];
-    }
-  }
-  if (lane == 0) f0[NY] = f.e;
-}
-// zero rows 0..NY of pencil p of a field in the transfer precision V
-template <int NY, typename V>
-__device__ __forceinline__ void pf_store_zero(V* __restrict__ F, size_t P, size_t p, int lane) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g = s * WAVE + lane;
-    if (g < L) { F[(size_t)(2 * g) * P + p] = vzero<V>(); F[(size_t)(2 * g + 1) * P + p] = vzero<V>(); }
-  }
-  if (lane == 0) F[(size_t)NY * P + p] = vzero<V>();
 }
 // real mean profile (nyp doubles)
 template <int NY>
@@ -809,22 +775,6 @@ __device__ __forceinline__ void pencil_k(const Args& A, int p, double& kx, doubl
   kz = kzs * A.beta;
 }
 
-template <int NY>
-__device__ __forceinline__ PFN<NY> smooth_apply(const PFN<NY>& f, const double* __restrict__ smy, double sz,
-                                                int lane) {
-  constexpr int L = PLay<NY>::L, S = PLay<NY>::S;
-  PFN<NY> r = f;
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    const int g = s * WAVE + lane;
-    if (g < L) {
-      r.a[s] = cscale(f.a[s], sz * smy[2 * g]);
-      r.b[s] = cscale(f.b[s], sz * smy[2 * g + 1]);
-    }
-  }
-  r.e = cscale(f.e, sz * smy[NY]);
-  return r;
-}
 
 // host-side helpers of the pencil launchers
 #define KMM_NY_DISPATCH(ny, ...) \
