@@ -4,11 +4,11 @@
 // polynomial-sigmoid factor
 // x sigma(1.702 x), chosen per network.
 //
-//   k_mlp_infer   inference on the matrix cores: v_mfma_f32_32x32x16_bf16
+//   k_mlp_infer   inference on the matrix cores: v_mfma_f32_16x16x32_bf16
 //                 with the weights as the A operand (staged once per block in
 //                 LDS, input index permuted so that each layer's accumulators
 //                 are the next layer's B operands) and the activations of
-//                 kT tiles of 32 points in registers; 8 wavefronts per block,
+//                 kT tiles of 16 points in registers; 8 wavefronts per block,
 //                 one block per CU, persistent over passes of 64 points.
 //   k_mlp_fb, k_mlp_wgrad, k_mlp_reduce   training: forward + backward, the
 //                 weight gradients and their sum (fixed order, no atomics)
@@ -32,7 +32,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
@@ -49,10 +48,10 @@ __host__ __device__ constexpr int w_off(int l) {
 __host__ __device__ constexpr int b_off(int l) { return w_off(l) + lay_out(l) * lay_in(l); }
 constexpr int kParams = w_off(kNL);
 
-// padded bf16 layout for the matrix cores: K padded to 32, N to 32, rows of
+// padded bf16 layout for the matrix cores: K padded to 32, N to 16, rows of
 // K + 8 elements
 __host__ __device__ constexpr int kin_pad(int l) { return l == 0 ? 32 : kH; }
-__host__ __device__ constexpr int nout_pad(int l) { return l == kNL - 1 ? 32 : kH; }
+__host__ __device__ constexpr int nout_pad(int l) { return l == kNL - 1 ? 16 : kH; }
 __host__ __device__ constexpr int wrow(int l) { return kin_pad(l) + 8; }
 __host__ __device__ constexpr int wb_off(int l) {
   int o = 0;
@@ -60,13 +59,13 @@ __host__ __device__ constexpr int wb_off(int l) {
   return o;
 }
 constexpr int kWb = wb_off(kNL);  // bf16 elements of the padded weights
-constexpr int kBias = 4 * kH + 32;
+constexpr int kBias = 4 * kH + 16;
 
 // activation: ReLU.  On the matrix-core path it is applied to the packed bf16
 // pair after rounding (a negative bf16 is a negative int16, so one
 // v_pk_max_i16 against 0 serves two activations; rounding and ReLU commute).
 // On gfx950 the vector ALU and the matrix cores do not overlap, so the
-// activation's instruction count sets most of inference time.
+// activation's instruction count sets a large part of inference time.
 __device__ __forceinline__ float act_f(float x) { return fmaxf(x, 0.0f); }
 __device__ __forceinline__ float act_df(float x) { return x > 0.0f ? 1.0f : 0.0f; }
 // GELU in the sigmoid form x sigma(1.702 x) (Hendrycks and Gimpel, "Gaussian
@@ -117,29 +116,20 @@ int mlp_param_count() { return kParams; }
 int mlp_wb_count() { return kWb; }
 
 // -------------------------------------------------------------- inference --
-// Layout for the matrix cores.  One v_mfma_f32_32x32x16_bf16 computes
-// D[m][n] = sum_k A[m][k] B[k][n] + C[m][n] with lane l holding A row l%32,
-// B column l%32, both at k = 8 (l/32) + i (i < 8), and D column l%32, rows
-// 8 (i/4) + 4 (l/32) + i%4 (i < 16).  Inference puts the weights in A (m =
-// output neuron) and the activations in B (n = point), so a lane's D values
-// 8 (j%2) .. 8 (j%2) + 7 of neuron tile j/2 are exactly the eight B values it
-// needs at k-step j of the next layer once the next layer's input index is
-// permuted:
-//   slot s = 16 j + 8 h + i  <->  neuron 16 j + 8 (i/4) + 4 h + i%4,
-// which exchanges bits 2 and 3.  The permutation is applied to the packed bf16
-// weights, so activations never leave registers between layers.  The first
-// layer's slots hold the features in the order that lets each half wavefront h
-// keep 2 h1 - h2 for the outputs it produces (h = 0 rows 0-3, h = 1 rows 4-5
-// of the last layer):
-//   slots 0-7 (h=0) h1[0..3], (h1-h2)[0..3]   16-23 (h=0) g[4..8], wall distance, 0, 0
-//   8-15 (h=1) h1[4,5], (h1-h2)[4,5], g[0..3] 24-31 (h=1) 0
-// Bound by issue: vector and matrix instructions do not overlap on gfx950, and
-// a pass of 64 points takes 4150 vector instructions of 4 cycles (3840 of them
-// the 512 activations' polynomial and rounding) and 224 products of 32.
-// Measured for 10.7 M points with ACT 2 at the 2.1 GHz held there: 1.79 ms;
-// 16x16x32 products with the activations one after another 1.87, the next
-// pass's loads issued early 1.96 (spills), one tile a wavefront with three or
-// four wavefronts a SIMD 1.79 and 1.85.
+// Layout for the matrix cores.  One v_mfma_f32_16x16x32_bf16 computes
+// D[m][n] = sum_k A[m][k] B[k][n] + C[m][n] with lane l holding A row l%16,
+// B column l%16, both at k = 8 (l/16) + i (i < 8), and D column l%16, rows
+// 4 (l/16) + i (i < 4).  Inference puts the weights in A (m = output neuron)
+// and the activations in B (n = point), so a lane's D values for neuron tiles
+// 2j and 2j+1 are exactly the eight B values it needs at k-step j of the next
+// layer once the next layer's input index is permuted:
+//   slot s = 32 j + 8 q + i  <->  neuron 32 j + 16 (i/4) + 4 q + i%4.
+// The permutation is applied to the packed bf16 weights, so activations never
+// leave registers between layers.  The first layer's slots hold the features
+// in the order that lets lanes q = 0, 1 keep 2 h1 - h2 for the outputs they
+// produce (rows 0-3 and 4-5 of the last layer):
+//   q=0: h1[0..3], (h1-h2)[0..3]     q=1: h1[4,5], (h1-h2)[4,5], g[0..3]
+//   q=2: g[4..8], wall distance, 0, 0     q=3: 0
 __host__ __device__ constexpr int feat_of_slot(int s) {
   return s < 4 ? 10 + s : s < 8 ? 12 + s : s < 10 ? 6 + s : s < 12 ? 10 + s : s < 21 ? s - 12 : s == 21 ? 9 : -1;
 }
@@ -147,18 +137,18 @@ __host__ __device__ constexpr int slot_of_feat(int k) {
   return k < 9 ? 12 + k : k == 9 ? 21 : k < 14 ? k - 10 : k < 16 ? k - 6 : k < 20 ? k - 12 : k - 10;
 }
 __host__ __device__ constexpr int neuron_of_slot(int s) {
-  return (s & ~12) | ((s & 4) << 1) | ((s & 8) >> 1);
+  return (s & ~31) | ((s & 4) << 2) | ((s & 24) >> 1) | (s & 3);
 }
 __host__ __device__ constexpr int slot_of_neuron(int k) {
-  return neuron_of_slot(k);
+  return (k & ~31) | ((k & 12) << 1) | ((k & 16) >> 2) | (k & 3);
 }
 // packed position of input index k of layer l
 __host__ __device__ constexpr int slot_of(int l, int k) { return l == 0 ? slot_of_feat(k) : slot_of_neuron(k); }
 // input index of packed slot s of layer l (-1: padding)
 __host__ __device__ constexpr int input_of(int l, int s) { return l == 0 ? feat_of_slot(s) : neuron_of_slot(s); }
 
-constexpr int kT = 2;             // 32-point tiles per wavefront pass (each weight read feeds kT products)
-constexpr int kChunk = 32 * kT;   // points per pass
+constexpr int kT = 4;             // 16-point tiles per wavefront pass (each weight read feeds kT products)
+constexpr int kChunk = 16 * kT;   // points per pass
 constexpr int kInferThreads = 512;  // 8 wavefronts: 2 per SIMD
 
 __device__ __forceinline__ float wall_feature(const MlpFieldIO& io, size_t p) {
@@ -174,60 +164,56 @@ __device__ __forceinline__ float field_feature(const MlpFieldIO& io, size_t p, i
   return io.h1[(size_t)(k - 16) * io.P + p] - io.h2[(size_t)(k - 16) * io.P + p];
 }
 
+// activation of two FP32 values, rounded to a packed bf16 pair: ReLU after
+// the rounding (ACT 0), GELU before it (ACT 1)
+template <int ACT>
+__device__ __forceinline__ unsigned act_pk(float a, float b) {
+  if constexpr (ACT == 1) {
+    const bf16x2 p = __builtin_convertvector(f32x2{gelu_f(a), gelu_f(b)}, bf16x2);
+    return __builtin_bit_cast(unsigned, p);
+  } else {
+    const bf16x2 p = __builtin_convertvector(f32x2{a, b}, bf16x2);  // one v_cvt_pk_bf16_f32
+    return __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(i16x2, p), i16x2{0, 0}));
+  }
+}
+
 // Eight values that an instruction stream may not reorder around: what was
 // asked for before is done for all eight first.
+template <bool ON>
 __device__ __forceinline__ void eight(float (&v)[8]) {
-  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+  if constexpr (ON)
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
 }
-// activation of eight FP32 values, rounded to packed bf16 pairs: ReLU after
-// the rounding (ACT 0), GELU before it (ACT 1, 2).  The eight go through
-// GELU's steps side by side; the compiler's own order saves registers and has
-// each instruction wait for the one before.
-template <int ACT>
-__device__ __forceinline__ u32x4 act_pk8(const float (&x)[8]) {
-  float y[8];
-  if constexpr (ACT == 1) {
+// gelup_f of eight values side by side, rounded to packed bf16 pairs; ORD
+// holds the compiler to that order (its own saves registers and has each
+// instruction wait for the one before)
+template <bool ORD>
+__device__ __forceinline__ u32x4 gelup_pk8(const float (&x)[8]) {
+  float t[8], u[8], y[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = __expf(-kGeluA * x[i]);
-    eight(y);
+  for (int i = 0; i < 8; ++i) t[i] = gelup_t(x[i]);
+  eight<ORD>(t);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = __builtin_amdgcn_rcpf(1.0f + y[i]);
-    eight(y);
+  for (int i = 0; i < 8; ++i) u[i] = t[i] * t[i];
+  eight<ORD>(u);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * y[i];
-  } else if constexpr (ACT == 2) {
-    float t[8], u[8];
+  for (int i = 0; i < 8; ++i) y[i] = fmaf(t[i], 6.0f, -15.0f);
+  eight<ORD>(y);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) t[i] = gelup_t(x[i]);
-    eight(t);
+  for (int i = 0; i < 8; ++i) u[i] = u[i] * t[i];
+  eight<ORD>(u);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) u[i] = t[i] * t[i];
-    eight(u);
+  for (int i = 0; i < 8; ++i) y[i] = fmaf(t[i], y[i], 10.0f);
+  eight<ORD>(y);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = fmaf(t[i], 6.0f, -15.0f);
-    eight(y);
+  for (int i = 0; i < 8; ++i) y[i] = u[i] * y[i];
+  eight<ORD>(y);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) u[i] = u[i] * t[i];
-    eight(u);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = fmaf(t[i], y[i], 10.0f);
-    eight(y);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = u[i] * y[i];
-    eight(y);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = x[i] * y[i];
-  }
+  for (int i = 0; i < 8; ++i) y[i] = x[i] * y[i];
   u32x4 o;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if constexpr (ACT == 0) {
-      const bf16x2 p = __builtin_convertvector(f32x2{x[2 * e], x[2 * e + 1]}, bf16x2);  // one v_cvt_pk_bf16_f32
-      o[e] = __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(i16x2, p), i16x2{0, 0}));
-    } else {
-      o[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{y[2 * e], y[2 * e + 1]}, bf16x2));
-    }
-  }
+  for (int e = 0; e < 4; ++e)
+    o[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{y[2 * e], y[2 * e + 1]}, bf16x2));
   return o;
 }
 
@@ -238,46 +224,86 @@ __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
   return __builtin_bit_cast(u32x4, o);
 }
 
-// One layer with KS input k-steps and 128 outputs, four neuron tiles of 32:
-// A operands (weights, rows of wr bf16) from LDS, each read once per pass,
-// three k-steps ahead, and used for kT point tiles; the bias enters as the
-// accumulator of the first k-step; outputs activated, rounded to bf16 and laid
-// out as the next layer's B operands.
-template <int KS, int ACT>
-__device__ __forceinline__ void mlp_layer(const u32x4 (&in)[KS][kT], u32x4 (&out)[8][kT], const __bf16* W, int wr,
-                                          const float* bias, int r32, int h) {
-  const __bf16* wl = W + r32 * wr + h * 8;  // this lane's A row in tile 0
-  const float* bl = bias + 4 * h;            // this lane's accumulator rows in tile 0
-  bf16x8 a[4];
+// One layer with KS input k-steps and 128 outputs, eight neuron tiles of 16:
+// A operands (weights, rows of wr bf16) from LDS, each read once per pass and
+// used for kT point tiles; the bias enters as the accumulator of the first
+// k-step; outputs activated, rounded to bf16 and laid out as the next layer's
+// B operands (tile nt fills elements 4 (nt%2) .. 4 (nt%2) + 3 of out[nt/2]).
+// Software pipelined: tile nt's products are interleaved with the activation
+// of tile nt-1 and with the weight reads of tile nt+1, so that neither waits
+// for the other's results.
+//
+// Bound by issue: vector and matrix instructions do not overlap on gfx950, and
+// a pass of 64 points takes 432 products of 16 cycles and, with ACT 2, about
+// 4000 vector instructions of 4 cycles (3840 of them the 512 activations'
+// polynomial and rounding).  ACT 2 therefore gains from eight activations
+// side by side (gelup_pk8), the others from the interleaving alone.  Measured
+// with ACT 0, 1, 2 (us; the closure's step is 192 x 129 x 192, 10.7 M points):
+//                                       10^6 rows       one row        closure's step
+//   this form                           101  206  181   8.6 15.7 15.2  950 1820 1640
+//   ACT 2's activations one by one      101  206  188   8.6 15.7 15.0  950 1820 1710
+//   32x32x16 products, not interleaved  112  211  179  10.1 17.2 17.3 1000 1820 1660
+// ORD, the order of the eight held (the field kernel), is 2 % there; one row
+// takes 16.0 with it, 15.2 without, so the row kernel leaves it to the compiler.
+template <int KS, int ACT, bool ORD>
+__device__ __forceinline__ void mlp_layer(const u32x4 (&in)[KS][kT], u32x4 (&out)[4][kT], const __bf16* W, int wr,
+                                          const float* bias, int r16, int kq) {
+  const __bf16* wl = W + r16 * wr + kq * 8;  // this lane's A row in tile 0
+  const float* bl = bias + 4 * kq;            // this lane's four accumulator rows in tile 0
+  f32x4 acc[2][kT];
+  bf16x8 a[2][KS];
+  f32x4 bb[2];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const bf16x8*>(wl + (q / KS) * 32 * wr + (q % KS) * 16);
+  for (int ks = 0; ks < KS; ++ks) a[0][ks] = *reinterpret_cast<const bf16x8*>(wl + ks * 32);
+  bb[0] = *reinterpret_cast<const f32x4*>(bl);
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    f32x16 acc[kT], b;
+  for (int nt = 0; nt <= 8; ++nt) {
+    if (nt < 7) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(bl + 32 * nt + 8 * g);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) b[4 * g + i] = b4[i];
+      for (int ks = 0; ks < KS; ++ks)
+        a[(nt + 1) & 1][ks] = *reinterpret_cast<const bf16x8*>(wl + (nt + 1) * 16 * wr + ks * 32);
+      bb[(nt + 1) & 1] = *reinterpret_cast<const f32x4*>(bl + (nt + 1) * 16);
     }
+    if (nt < 8) {
+      const f32x4 b4 = bb[nt & 1];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int q = nt * KS + ks, n3 = q + 3;
-      if (n3 < 4 * KS) a[n3 & 3] = *reinterpret_cast<const bf16x8*>(wl + (n3 / KS) * 32 * wr + (n3 % KS) * 16);
+      for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int t = 0; t < kT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q & 3], __builtin_bit_cast(bf16x8, in[ks][t]),
-                                                         ks == 0 ? b : acc[t], 0, 0, 0);
+        for (int t = 0; t < kT; ++t)
+          acc[nt & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a[nt & 1][ks], __builtin_bit_cast(bf16x8, in[ks][t]), ks == 0 ? b4 : acc[nt & 1][t], 0, 0, 0);
     }
+    if (nt > 0) {
+      const int m = nt - 1;
 #pragma unroll
-    for (int t = 0; t < kT; ++t)
+      for (int t = 0; t < kT; t += 2) {
+        if constexpr (ACT == 2) {
+          float x[8];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float x[8];
+          for (int i = 0; i < 8; ++i) x[i] = acc[m & 1][t + i / 4][i % 4];
+          const u32x4 y = gelup_pk8<ORD>(x);
+          out[m >> 1][t][2 * (m & 1)] = y[0];
+          out[m >> 1][t][2 * (m & 1) + 1] = y[1];
+          out[m >> 1][t + 1][2 * (m & 1)] = y[2];
+          out[m >> 1][t + 1][2 * (m & 1) + 1] = y[3];
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = acc[t][8 * j + i];
-        out[2 * nt + j][t] = act_pk8<ACT>(x);
+          for (int q = t; q < t + 2; ++q) {
+            out[m >> 1][q][2 * (m & 1)] = act_pk<ACT>(acc[m & 1][q][0], acc[m & 1][q][1]);
+            out[m >> 1][q][2 * (m & 1) + 1] = act_pk<ACT>(acc[m & 1][q][2], acc[m & 1][q][3]);
+          }
+        }
       }
+    }
+    if (nt > 0 && nt < 8) {
+      // one product, then its share of the vector work
+#pragma unroll
+      for (int i = 0; i < KS * kT; ++i) {
+        if (i <= KS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 64 / (KS * kT) > 4 ? 64 / (KS * kT) : 4, 0);
+      }
+    }
     // keep each stage's registers from being hoisted into the previous one
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -297,12 +323,15 @@ __global__ __launch_bounds__(kInferThreads) void k_mlp_infer(int n, const float*
   float* sxs = sb + kBias;                                  // input scale per slot [32]
   float* sxo = sxs + 32;                                    // input shift per slot [32]
   const int tid = threadIdx.x, lane = tid & 63;
+  // 2 h1 - h2 of the outputs this lane produces, kept here between the ends of
+  // a pass: in registers ACT 2 spills 88 bytes a lane (1.73 against 1.64 ms)
+  f32x4* exl = reinterpret_cast<f32x4*>(sxo + 32) + tid;
   {
     const uint4* src = reinterpret_cast<const uint4*>(wb);
     uint4* dst = reinterpret_cast<uint4*>(sw);
     for (int e = tid; e < kWb / 8; e += blockDim.x) dst[e] = src[e];
   }
-  // biases: layer l at 128 l (the last layer's 16 padded entries at 512)
+  // biases: layer l at 128 l (the last layer's padded entries at 512)
   for (int l = 0; l < kNL; ++l)
     for (int j = tid; j < nout_pad(l); j += blockDim.x) sb[128 * l + j] = (j < lay_out(l)) ? par[b_off(l) + j] : 0.0f;
   if (tid < 32) {
@@ -313,118 +342,111 @@ __global__ __launch_bounds__(kInferThreads) void k_mlp_infer(int n, const float*
   __syncthreads();
   const float* mu_y = norm + 2 * kIn;
   const float* sd_y = norm + 2 * kIn + kOut;
-  const int r32 = lane & 31, h = lane >> 5;
+  const int r16 = lane & 15, kq = lane >> 4;
   const int npass = (n + kChunk - 1) / kChunk;
   const int nwave = gridDim.x * (blockDim.x >> 6);
   for (int c = blockIdx.x * (blockDim.x >> 6) + (tid >> 6); c < npass; c += nwave) {
     const int p0 = c * kChunk;
-    u32x4 x0[2][kT];
-    float ex[kT][4];  // 2 h1 - h2 of the outputs this lane produces
+    u32x4 x0[1][kT];
     // all of the pass's loads first, then one wait.  Every load instruction
-    // reads one array for the whole wavefront (rows chosen per half, always in
-    // range; h = 1 discards the repeats): A = h1 rows 4 h + j, B = h2
-    // likewise, G = g rows 4 + j (h = 0) or j (h = 1).
-    float A[kT][4], B[kT][4], G[kT][5], C[kT][8];
+    // reads one array for the whole wavefront (rows chosen per lane group,
+    // always in range; the values a group does not need are discarded):
+    // A = h1 rows 4q + j (q = 0: 0-3, q = 1: 4-5), B = h2 likewise,
+    // G = g rows 4 (q >= 2) + j (q = 1: 0-3, q >= 2: 4-8).
+    float A[kT][4], B[kT][4], G[kT][5];
     double yc[kT];
     const unsigned P = FIELD ? (unsigned)io.P : 0u;
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
-      const unsigned p = (unsigned)min(p0 + 32 * t + r32, n - 1);
+      const unsigned p = (unsigned)min(p0 + 16 * t + r16, n - 1);
       if (FIELD) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const unsigned o = (unsigned)min(4 * h + j, 5) * P + p;
-          A[t][j] = io.h1[o];
-          B[t][j] = io.h2[o];
+          const unsigned row = (unsigned)min(4 * kq + j, 5);
+          A[t][j] = io.h1[row * P + p];
+          B[t][j] = io.h2[row * P + p];
         }
 #pragma unroll
-        for (int j = 0; j < 5; ++j) G[t][j] = io.g[(unsigned)(h ? j : 4 + j) * P + p];
+        for (int j = 0; j < 5; ++j) G[t][j] = io.g[(unsigned)min((kq >= 2 ? 4 : 0) + j, 8) * P + p];
         yc[t] = io.ycoord[p / (unsigned)io.plane_pts];
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const int k = feat_of_slot(8 * h + j), k1 = feat_of_slot(16 + 8 * h + j);
-          const float x = X[(size_t)p * kIn + k];
+          const int k = feat_of_slot(8 * kq + j);
+          const float x = X[(size_t)p * kIn + (k < 0 ? 0 : k)];
           if (j < 4) A[t][j] = x;
           else B[t][j - 4] = x;
-          C[t][j] = X[(size_t)p * kIn + (k1 < 0 ? 0 : k1)];
         }
       }
     }
+    const bool q0 = kq == 0, q1 = kq == 1;
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
-      float v[8], v1[8];
+      float v[8];
       if (FIELD) {
+        // slots of this lane's group: q=0 h1[0..3], h1[0..3]-h2[0..3];
+        // q=1 h1[4,5], h1[4,5]-h2[4,5], g[0..3]; q=2 g[4..8], wall, 0, 0
         const float wall = (float)(1.0 - fabs(yc[t]) / io.half);
         float d[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          d[i] = A[t][i] - B[t][i];  // the last step's change, in FP32
-          ex[t][i] = A[t][i] + d[i];
-        }
-        v[0] = A[t][0];
-        v[1] = A[t][1];
-        v[2] = h ? d[0] : A[t][2];
-        v[3] = h ? d[1] : A[t][3];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[4 + i] = h ? G[t][i] : d[i];
-#pragma unroll
-        for (int i = 0; i < 5; ++i) v1[i] = G[t][i];  // h = 1: slots of scale 0
-        v1[5] = wall;
-        v1[6] = v1[7] = 0.0f;
+        for (int i = 0; i < 4; ++i) d[i] = A[t][i] - B[t][i];  // the last step's change, in FP32
+        exl[t * kInferThreads] = f32x4{A[t][0] + d[0], A[t][1] + d[1], A[t][2] + d[2], A[t][3] + d[3]};
+        v[0] = q0 || q1 ? A[t][0] : G[t][0];
+        v[1] = q0 || q1 ? A[t][1] : G[t][1];
+        v[2] = q0 ? A[t][2] : q1 ? d[0] : G[t][2];
+        v[3] = q0 ? A[t][3] : q1 ? d[1] : G[t][3];
+        v[4] = q0 ? d[0] : q1 ? G[t][0] : G[t][4];
+        v[5] = q0 ? d[1] : q1 ? G[t][1] : wall;
+        v[6] = q0 ? d[2] : q1 ? G[t][2] : 0.0f;
+        v[7] = q0 ? d[3] : q1 ? G[t][3] : 0.0f;
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           v[i] = A[t][i];
           v[4 + i] = B[t][i];
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v1[i] = C[t][i];
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        v[i] = fmaf(v[i], sxs[8 * h + i], sxo[8 * h + i]);
-        v1[i] = h ? 0.0f : fmaf(v1[i], sxs[16 + i], sxo[16 + i]);
-      }
+      for (int i = 0; i < 8; ++i) v[i] = fmaf(v[i], sxs[8 * kq + i], sxo[8 * kq + i]);
       x0[0][t] = pack8(v);
-      x0[1][t] = pack8(v1);
     }
-    u32x4 a1[8][kT], a2[8][kT];
-    mlp_layer<2, ACT>(x0, a1, sw + wb_off(0), wrow(0), sb, r32, h);
-    mlp_layer<8, ACT>(a1, a2, sw + wb_off(1), wrow(1), sb + 128, r32, h);
-    mlp_layer<8, ACT>(a2, a1, sw + wb_off(2), wrow(2), sb + 256, r32, h);
-    mlp_layer<8, ACT>(a1, a2, sw + wb_off(3), wrow(3), sb + 384, r32, h);
+    u32x4 a1[4][kT], a2[4][kT];
+    mlp_layer<1, ACT, FIELD>(x0, a1, sw + wb_off(0), wrow(0), sb, r16, kq);
+    mlp_layer<4, ACT, FIELD>(a1, a2, sw + wb_off(1), wrow(1), sb + 128, r16, kq);
+    mlp_layer<4, ACT, FIELD>(a2, a1, sw + wb_off(2), wrow(2), sb + 256, r16, kq);
+    mlp_layer<4, ACT, FIELD>(a1, a2, sw + wb_off(3), wrow(3), sb + 384, r16, kq);
     // output layer: one neuron tile (rows 0-5 used)
-    f32x16 acc[kT];
+    f32x4 acc[kT];
     {
       const __bf16* W = sw + wb_off(4);
-      f32x16 b = {};
-      const f32x4 b4 = *reinterpret_cast<const f32x4*>(sb + 512 + 4 * h);
+      const f32x4 b4 = *reinterpret_cast<const f32x4*>(sb + 512 + 4 * kq);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) b[i] = b4[i];
-#pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(W + r32 * wrow(4) + ks * 16 + h * 8);
+      for (int ks = 0; ks < 4; ++ks) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(W + r16 * wrow(4) + ks * 32 + kq * 8);
 #pragma unroll
         for (int t = 0; t < kT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, a2[ks][t]), ks == 0 ? b : acc[t],
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, a2[ks][t]), ks == 0 ? b4 : acc[t],
                                                            0, 0, 0);
       }
     }
-    const int nout = h ? 2 : 4;
+    if (kq < 2) {
+      const int nout = kq == 0 ? 4 : 2;
 #pragma unroll
-    for (int t = 0; t < kT; ++t) {
-      const int p = p0 + 32 * t + r32;
-      if (p < n) {
+      for (int t = 0; t < kT; ++t) {
+        const int p = p0 + 16 * t + r16;
+        if (p < n) {
+          f32x4 ex = {};
+          if (FIELD) ex = exl[t * kInferThreads];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int col = 4 * h + i;
-          if (i < nout) {
-            const float yv = acc[t][i] * sd_y[col] + mu_y[col];
-            // the closure network predicts the correction to linear
-            // extrapolation of the two previous steps: out = 2 h1 - h2 + y
-            if (FIELD) io.out[(size_t)col * io.P + p] = ex[t][i] + yv;
-            else Y[(size_t)p * kOut + col] = yv;
+          for (int i = 0; i < 4; ++i) {
+            const int col = 4 * kq + i;
+            if (i < nout) {
+              const float yv = acc[t][i] * sd_y[col] + mu_y[col];
+              // the closure network predicts the correction to linear
+              // extrapolation of the two previous steps: out = 2 h1 - h2 + y
+              if (FIELD) io.out[(size_t)col * io.P + p] = ex[i] + yv;
+              else Y[(size_t)p * kOut + col] = yv;
+            }
           }
         }
       }
@@ -432,7 +454,10 @@ __global__ __launch_bounds__(kInferThreads) void k_mlp_infer(int n, const float*
   }
 }
 
-size_t mlp_infer_lds() { return (size_t)kWb * 2 + (size_t)kBias * 4 + 64 * 4; }
+static_assert((kWb * 2 + kBias * 4 + 64 * 4) % 16 == 0, "LDS layout");
+constexpr size_t mlp_infer_lds(bool field) {
+  return (size_t)kWb * 2 + (size_t)kBias * 4 + 64 * 4 + (field ? (size_t)kInferThreads * kT * 16 : 0);
+}
 
 static int device_cus() {
   int dev = 0, cus = 0;
@@ -452,11 +477,11 @@ static hipError_t mlp_infer_launch_a(int n, const float* X, float* Y, const MlpF
   static bool attr = false;  // > 64 KB of dynamic LDS (160 KB per CU on gfx950)
   if (!attr) {
     hipError_t e = hipFuncSetAttribute((const void*)k_mlp_infer<FIELD, ACT>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlp_infer_lds());
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)mlp_infer_lds(FIELD));
     if (e != hipSuccess) return e;
     attr = true;
   }
-  hipLaunchKernelGGL((k_mlp_infer<FIELD, ACT>), dim3(blocks), dim3(kInferThreads), mlp_infer_lds(), s, n, X, Y, io,
+  hipLaunchKernelGGL((k_mlp_infer<FIELD, ACT>), dim3(blocks), dim3(kInferThreads), mlp_infer_lds(FIELD), s, n, X, Y, io,
                      static_cast<const __bf16*>(wb), par, norm);
   return hipGetLastError();
 }
