@@ -247,7 +247,7 @@ extern "C" int kmm_mlp_train(kmm_mlp* n, int npts, const float* X, const float* 
 }
 
 // Adam steps on samples already on the device (dX [npts][22], dT [npts][6]),
-// queued on stream s without host synchronisation: step k uses the k-th
+// queued on stream s once the device is idle (not waited for): step k uses the k-th
 // consecutive block of `batch` samples (cycling), so the samples must come
 // in random order (kmm_poly_samples' sampler draws them so).  Used by the
 // channel to retrain the closure on pairs drawn inside audit windows.
@@ -255,6 +255,9 @@ int kmm_mlp_train_device(kmm_mlp* n, int npts, const float* dX, const float* dT,
                          hipStream_t s) {
   if (!n || npts <= 0 || !dX || !dT || steps <= 0 || batch <= 0 || batch > npts || !(lr > 0.0f))
     return mfail(KMM_E_ARG, "bad argument");
+  // the network may serve several channels: steps already queued on the other
+  // channels' streams still run with the weights as they are now
+  MHIP(hipDeviceSynchronize());
   int r;
   if ((r = grow(&n->ws, &n->capW, kmm::mlp_train_ws(batch)))) return r;
   const int nblocks = npts / batch;
