@@ -44,7 +44,13 @@ static int grow(float** p, size_t* cap, size_t n) {
   if (n <= *cap) return KMM_OK;
   if (*p) hipFree(*p);
   *p = nullptr;
-  MHIP(hipMalloc((void**)p, n * sizeof(float)));
+  *cap = 0;
+  const hipError_t e = hipMalloc((void**)p, n * sizeof(float));
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();  // reported here, not by the next launch
+    return mfail(KMM_E_HIP, std::string("network buffers: ") + hipGetErrorString(e));
+  }
   *cap = n;
   return KMM_OK;
 }
