@@ -309,7 +309,6 @@ hipError_t launch_pencil_step(int ny, const PencilArgs& a, hipStream_t s);
 hipError_t launch_pencil_startup(int ny, const PencilArgs& a, hipStream_t s);
 hipError_t launch_pencil_finish(int ny, const PencilArgs& a, hipStream_t s);
 hipError_t launch_plane(const PlaneArgs& a, hipStream_t s);
-hipError_t launch_plane_fwd_only(const PlaneArgs& a, hipStream_t s);
 // ev[0..3] recorded after k_zinv, k_ibdrag, k_xplane, k_zfwd
 hipError_t launch_plane_timed(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev);
 // one step of nmem channels of the same size in one launch per stage: dA

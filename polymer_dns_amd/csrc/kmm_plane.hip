@@ -1131,44 +1131,42 @@ static hipError_t poly_plane_impl(const PolyPlaneArgs& pa, hipStream_t s) {
 }
 
 template <int MX, int MZ, int NFIN, int NFOUT, typename V>
-static hipError_t plane_impl(const PlaneArgs& a, hipStream_t s, bool inverse_part, hipEvent_t* ev) {
-  if (inverse_part) {
-    launch_zinv<MZ, NFIN, V>(a, s);
-    if (ev) hipEventRecord(ev[0], s);
-    if (a.nsrc > 0)
-      hipLaunchKernelGGL((k_ibdrag<MX, V>), dim3((a.nsrc + 3) / 4), dim3(256), 0, s, a);
-    if (ev) hipEventRecord(ev[1], s);
-    constexpr int WPB = 4;
-    const size_t xlds = xfft_lds<MX, V>(WPB, xplane_lines<MX, NFIN, NFOUT>());
-    if (a.tune == 1)
-      hipLaunchKernelGGL((k_xplane<MX, NFIN, NFOUT, WPB, V, 1>), dim3(a.nyp * (a.mz / (2 * WPB))), dim3(WPB * 64),
-                         xlds, s, a);
-    else
-      hipLaunchKernelGGL((k_xplane<MX, NFIN, NFOUT, WPB, V, 0>), dim3(a.nyp * (a.mz / (2 * WPB))), dim3(WPB * 64),
-                         xlds, s, a);
-    if (ev) hipEventRecord(ev[2], s);
-  }
+static hipError_t plane_impl(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev) {
+  launch_zinv<MZ, NFIN, V>(a, s);
+  if (ev) hipEventRecord(ev[0], s);
+  if (a.nsrc > 0)
+    hipLaunchKernelGGL((k_ibdrag<MX, V>), dim3((a.nsrc + 3) / 4), dim3(256), 0, s, a);
+  if (ev) hipEventRecord(ev[1], s);
+  constexpr int WPB = 4;
+  const size_t xlds = xfft_lds<MX, V>(WPB, xplane_lines<MX, NFIN, NFOUT>());
+  if (a.tune == 1)
+    hipLaunchKernelGGL((k_xplane<MX, NFIN, NFOUT, WPB, V, 1>), dim3(a.nyp * (a.mz / (2 * WPB))), dim3(WPB * 64),
+                       xlds, s, a);
+  else
+    hipLaunchKernelGGL((k_xplane<MX, NFIN, NFOUT, WPB, V, 0>), dim3(a.nyp * (a.mz / (2 * WPB))), dim3(WPB * 64),
+                       xlds, s, a);
+  if (ev) hipEventRecord(ev[2], s);
   launch_zfwd<MZ, NFOUT, V>(a, s);
   if (ev) hipEventRecord(ev[3], s);
   return hipGetLastError();
 }
 
 template <int MX, int MZ>
-static hipError_t plane_dispatch_f(const PlaneArgs& a, hipStream_t s, bool inv, hipEvent_t* ev) {
+static hipError_t plane_dispatch_f(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev) {
   if (a.mixed) {
-    if (a.nfin == 6 && a.nfout == 3) return plane_impl<MX, MZ, 6, 3, float2>(a, s, inv, ev);
-    if (a.nfin == 9 && a.nfout == 4) return plane_impl<MX, MZ, 9, 4, float2>(a, s, inv, ev);
+    if (a.nfin == 6 && a.nfout == 3) return plane_impl<MX, MZ, 6, 3, float2>(a, s, ev);
+    if (a.nfin == 9 && a.nfout == 4) return plane_impl<MX, MZ, 9, 4, float2>(a, s, ev);
   } else {
-    if (a.nfin == 6 && a.nfout == 3) return plane_impl<MX, MZ, 6, 3, double2>(a, s, inv, ev);
-    if (a.nfin == 9 && a.nfout == 4) return plane_impl<MX, MZ, 9, 4, double2>(a, s, inv, ev);
+    if (a.nfin == 6 && a.nfout == 3) return plane_impl<MX, MZ, 6, 3, double2>(a, s, ev);
+    if (a.nfin == 9 && a.nfout == 4) return plane_impl<MX, MZ, 9, 4, double2>(a, s, ev);
   }
   return hipErrorInvalidValue;
 }
 
-static hipError_t plane_dispatch(const PlaneArgs& a, hipStream_t s, bool inv, hipEvent_t* ev) {
+static hipError_t plane_dispatch(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev) {
   if (a.nxh % 8 != 0) return hipErrorInvalidValue;
 #define KMM_PLANE_CASE(X, Zz) \
-  if (a.mx == X && a.mz == Zz) return plane_dispatch_f<X, Zz>(a, s, inv, ev);
+  if (a.mx == X && a.mz == Zz) return plane_dispatch_f<X, Zz>(a, s, ev);
   KMM_PLANE_CASE(48, 48)
   KMM_PLANE_CASE(96, 48)
   KMM_PLANE_CASE(96, 96)
@@ -1312,10 +1310,7 @@ hipError_t launch_closure_fwd(const PolyPlaneArgs& a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_plane(const PlaneArgs& a, hipStream_t s) { return plane_dispatch(a, s, true, nullptr); }
-hipError_t launch_plane_timed(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev) {
-  return plane_dispatch(a, s, true, ev);
-}
-hipError_t launch_plane_fwd_only(const PlaneArgs& a, hipStream_t s) { return plane_dispatch(a, s, false, nullptr); }
+hipError_t launch_plane(const PlaneArgs& a, hipStream_t s) { return plane_dispatch(a, s, nullptr); }
+hipError_t launch_plane_timed(const PlaneArgs& a, hipStream_t s, hipEvent_t* ev) { return plane_dispatch(a, s, ev); }
 
 }  // namespace kmm
