@@ -452,8 +452,8 @@ int kmm_write_flowfield(kmm_ctx* ctx, const char* dir, int it, int iprnfrq);
 
 /* Autotuner (no reference counterpart; the role of FFTW's PATIENT planning,
  * solvers.f90:2057-2069): occupancy variants of the pencil step kernel and of
- * the x-plane kernel (0: the compiler's register budget, 1: one more wave per
- * SIMD) are timed over `steps` steps on a twin of the context (same
+ * the x-plane kernel (0: the form and occupancy that the size's rule picks, 1:
+ * another number of waves per SIMD) are timed over `steps` steps on a twin of the context (same
  * configuration, geometry, tracers and state; the context itself does not
  * advance) and the faster of each is kept.  ms (or NULL) receives
  * {pencil v0, pencil v1, xplane v0, xplane v1} in ms per step. */

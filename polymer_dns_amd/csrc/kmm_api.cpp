@@ -1453,7 +1453,7 @@ static bool steady(const kmm_ctx* c, int k) {
   if (c->audit_w >= 0) return false;
   if (c->poly_capture) return false;                     // capture bookkeeping runs per launch
   if (c->npart > 0 && c->part_state != 2) return false;
-  if (inertial(c)) return false;  // per-step copies of the old fields and buffer swaps
+  if (inertial(c)) return false;  // the old fields' buffers change places every step
   if (c->nsrc > 0 && c->it < c->cfg.perturbtime + 1) return false;
   if (c->scsrc) {  // the source window must not open or close inside the graph
     const int a = c->it + 1, b = c->it + k, s0 = c->cfg.src_start, s1 = c->cfg.src_stop;

@@ -80,15 +80,6 @@ __device__ __forceinline__ double shdn1(double v) { return dpp<DPP_WAVE_SHL1>(v)
 __device__ __forceinline__ double2 shdn1(double2 v) { return dpp<DPP_WAVE_SHL1>(v); }
 __device__ __forceinline__ double shup1(double v) { return dpp<DPP_WAVE_SHR1>(v); }
 __device__ __forceinline__ double2 shup1(double2 v) { return dpp<DPP_WAVE_SHR1>(v); }
-
-__device__ __forceinline__ double shdn(double v, int off) { return __shfl_down(v, off, WAVE); }
-__device__ __forceinline__ double shup(double v, int off) { return __shfl_up(v, off, WAVE); }
-__device__ __forceinline__ double2 shdn(double2 v, int off) {
-  return make_double2(__shfl_down(v.x, off, WAVE), __shfl_down(v.y, off, WAVE));
-}
-__device__ __forceinline__ double2 shup(double2 v, int off) {
-  return make_double2(__shfl_up(v.x, off, WAVE), __shfl_up(v.y, off, WAVE));
-}
 __device__ __forceinline__ double bcast(double v, int src) { return rdlane(v, src); }
 __device__ __forceinline__ double2 bcast(double2 v, int src) { return rdlane(v, src); }
 

@@ -1,8 +1,7 @@
 // Learned polymer-stress closure: a 22 -> 4 x 128 -> 6 multilayer
 // perceptron with bfloat16 weights and FP32 accumulation (no reference
-// counterpart); hidden activation ReLU, or GELU with a sigmoid or a
-// polynomial-sigmoid factor
-// x sigma(1.702 x), chosen per network.
+// counterpart); hidden activation ReLU, GELU as x sigma(1.702 x), or GELU with
+// a polynomial in the sigmoid's place, chosen per network.
 //
 //   k_mlp_infer   inference on the matrix cores: v_mfma_f32_16x16x32_bf16
 //                 with the weights as the A operand (staged once per block in
