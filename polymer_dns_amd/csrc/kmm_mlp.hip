@@ -63,7 +63,7 @@ constexpr int kBias = 4 * kH + 16;
 // activation: ReLU.  On the matrix-core path it is applied to the packed bf16
 // pair after rounding (a negative bf16 is a negative int16, so one
 // v_pk_max_i16 against 0 serves two activations; rounding and ReLU commute).
-// On gfx950 the vector ALU and the matrix cores do not overlap, so the
+// On gfx950 the vector ALU and the matrix cores hardly overlap, so the
 // activation's instruction count sets a large part of inference time.
 __device__ __forceinline__ float act_f(float x) { return fmaxf(x, 0.0f); }
 __device__ __forceinline__ float act_df(float x) { return x > 0.0f ? 1.0f : 0.0f; }
@@ -232,11 +232,12 @@ __device__ __forceinline__ u32x4 pack8(const float (&v)[8]) {
 // of tile nt-1 and with the weight reads of tile nt+1, so that neither waits
 // for the other's results.
 //
-// Bound by issue: vector and matrix instructions do not overlap on gfx950, and
-// a pass of 64 points takes 432 products of 16 cycles and, with ACT 2, about
-// 4000 vector instructions of 4 cycles (3840 of them the 512 activations'
-// polynomial and rounding).  ACT 2 therefore gains from eight activations
-// side by side (gelup_pk8), the others from the interleaving alone.  Measured
+// Bound by issue: vector and matrix instructions hardly overlap on gfx950, and
+// a pass of 64 points takes 432 products of 16 cycles and, with ACT 2, 4265
+// vector instructions of 4 (3840 of them the 512 activations' polynomial and
+// rounding), together 112 % of its cycles (counted).  ACT 2 therefore gains
+// from eight activations side by side (gelup_pk8), the others from the
+// interleaving alone.  Measured
 // with ACT 0, 1, 2 (us; the closure's step is 192 x 129 x 192, 10.7 M points):
 //                                       10^6 rows       one row        closure's step
 //   this form                           101  206  181   8.6 15.7 15.2  950 1820 1640

@@ -613,7 +613,7 @@ __device__ __forceinline__ void pair_write(V* buf, int g, const typename Scal<V>
   xline_write<MX, V>(buf, g, p, lane);
 }
 
-// The 18 pair transforms of a row: field ids >= 0 index the z-stage outputs
+// The 21 pair transforms of a row: field ids >= 0 index the z-stage outputs
 // (dz u 0-2, dy u 3-5, C 6-11, dz C 12-17, dy C 18-23), ids < 0 the velocity
 // intermediates (-1 - f); dx = multiply by i alpha k first.
 struct PairSpec {
@@ -819,7 +819,7 @@ struct PolyRow {
 };
 
 // Two waves per SIMD (256 registers: FP64 spills 52 bytes a lane at MX = 288,
-// 208 at 384; one wave per SIMD without spills is slower, the LDS of two
+// 276 at 384; one wave per SIMD without spills is slower, the LDS of two
 // blocks a CU allows no third), FP32 rows of 288 and 384 points three.
 template <int MX, typename V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MX >= 288 && sizeof(V) == 8 ? 3 : 2)))
